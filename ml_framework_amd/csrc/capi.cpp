@@ -231,7 +231,7 @@ int convT_fwd_impl(const float* X, const float* Wt, float* out, int batch, int C
     int Hout, Wout;
     SEERA_TRY(convT_dims(Hin, Win, KH, KW, sh, sw, ph, pw, &Hout, &Wout));
     SEERA_TRY(check_ptrs(batch > 0, X, Wt, out));
-    return conv_dgrad(X, Wt, out, batch, Cin, Hin, Win, Cout, Hout, Wout, KH, KW, sh, sw, ph, pw,
+    return convT_fwd(X, Wt, out, batch, Cin, Hin, Win, Cout, Hout, Wout, KH, KW, sh, sw, ph, pw,
                       st);
 }
 
@@ -246,10 +246,7 @@ int convT_bwd_impl(const float* Wt, const float* X, const float* dY, float* dX, 
                          batch > 0 ? dX : dW));
     // dX = conv2d(dY, W viewed as [F = Cin, C = Cout, KH, KW]); its output
     // extent (Hout + 2ph - KH)/sh + 1 equals Hin exactly.
-    SEERA_TRY(conv_fwd(dY, Wt, dX, batch, Cout, Hout, Wout, Cin, KH, KW, sh, sw, ph, pw, st));
-    // dW[ci, co, kh, kw] = sum X[b, ci, hi, wi] dY[b, co, hi*sh-ph+kh, wi*sw-pw+kw]:
-    // the conv weight gradient with X in the role of dY and dY in that of X.
-    return conv_wgrad(X, dY, dW, nullptr, batch, Cout, Hout, Wout, Cin, KH, KW, sh, sw, ph, pw, st);
+    return convT_bwd(dY, Wt, X, dX, dW, batch, Cin, Hin, Win, Cout, Hout, Wout, KH, KW, sh, sw, ph, pw, st);
 }
 
 template <class F>

@@ -15,6 +15,7 @@
 //            = conv2d dW   (convolution.cu:268-366, 431-452)
 //            = convT dW    (upsampling.cu:202-301, 354-374; roles of X, dY swapped)
 #include "conv_band.h"
+#include "conv_packed.h"
 #include "gather.h"
 #include "kernels.h"
 #include "plan.h"
@@ -391,6 +392,75 @@ unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 25
 
 namespace {
 
+// Whether a pass runs on operands packed to fp16 (conv_packed.hip) or on the
+// kernels that read fp32 NCHW rows directly (conv_band.hip and the streaming
+// kernels). Packing costs one pass over the operands and pays where the direct
+// kernels read every value several times over (many filters), have few blocks
+// (many channels on small images), widen rows that are not float4s first, or
+// miss their fast shapes; it does not where a layer of few channels on large
+// aligned images is bound by reading its input once. Measured direct -> packed,
+// us, N x C x H x W -> F:
+//   3x3 s1  64x256x14x14 -> 256  fwd 68 -> 33, bwd 151 -> 66
+//           64x512x7x7 -> 512    fwd 67 -> 38, bwd 224 -> 76
+//           64x128x32x32 -> 128  fwd 68 -> 38, bwd 116 -> 98
+//           64x64x56x56 -> 128   fwd 51 -> 80, bwd 131 -> 175 (direct)
+//           64x128x32x32 -> 64   fwd 38 -> 29, bwd 62 -> 71 (bwd direct)
+//           64x32x8x8 -> 64      fwd 13 -> 13, bwd 36 -> 19
+//   3x3 s2  64x128x28x28 -> 256  fwd 43 -> 27, bwd 117 -> 61
+//   1x1     64x256x16x16 -> 256  fwd 37 -> 19, bwd 101 -> 36
+//           64x128x56x56 -> 64   fwd 56 -> 64, bwd 96 -> 104 (direct)
+//   5x5 s1  32x64x28x28 -> 64    fwd 164 -> 23, bwd 569 -> 54
+// The space-to-depth form of a first layer (few channels, large kernel, stride
+// 2) keeps its own path below.
+bool s2d_layer(int C, int R, int S, int sh, int sw) { return s2d_applies(R, S, sh, sw) && C <= 8; }
+
+bool packed_fwd_pays(int C, int W, int F, int R, int S, int sh, int sw, int ph, int pw) {
+    if (s2d_layer(C, R, S, sh, sw)) return false;
+    // 4 x 4 at stride 2 has a direct kernel (conv_stride2.hip): 32x64x16x16 ->
+    // 64 11 -> 16 us; other channel counts 16x128x64x64 -> 128 58 -> 32.
+    if (R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && (C == 32 || C == 64) && W % 4 == 0)
+        return false;
+    // Channels that are not a multiple of 8 (first layers): 39x3x28x28 -> 32
+    // 26 -> 13, 8x3x224x224 -> 64 71 -> 50.
+    if (W % 4 != 0 || C % 8 != 0 || R * S > 16 || sh > 1 || sw > 1) return true;
+    if (R * S == 1) return F >= 128 && (int64_t)C * F >= 128 * 128;
+    return C > 64;
+}
+
+bool packed_bwd_pays(int B, int C, int H, int W, int F, int R, int S, int sh, int sw, int ph, int pw) {
+    if (s2d_layer(C, R, S, sh, sw)) return false;
+    const int Wo = (W + 2 * pw - S) / sw + 1;
+    const int64_t pixels = (int64_t)B * H * W;
+    if (W % 4 != 0 || Wo % 4 != 0 || R * S > 16) return true;
+    // Few pixels: the direct kernels leave most CUs without a block, whatever
+    // the channels (16x32x32x32 -> 32 36 -> 24; at 64x64x28x28 -> 64, 50 k
+    // pixels, 41 -> 43). Channels not a multiple of 8: 111x3x28x28 -> 8 (87 k)
+    // 52 -> 44, 110x3x64x64 -> 8 80 -> 110.
+    if (pixels < 40000 || (C % 8 != 0 && pixels < 100000)) return true;
+    // (4 x 4 at stride 2, direct: conv_phase2.hip and conv_wgrad_s2.hip;
+    // 16x128x64x64 -> 128 50 -> 57)
+    if (R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && F % 32 == 0 && F <= 128 && W % 8 == 0)
+        return false;
+    if (sh > 1 || sw > 1) return true;
+    if (R * S == 1) return F >= 128;
+    return C >= 128 && F >= 128;
+}
+
+// ConvTranspose2D of 4 x 4 at stride 2 keeps its direct kernels
+// (conv_phase2.hip, conv_stride2.hip) on the channel counts they take:
+// 64x128x28x28 -> 64 fwd 33 -> 55, bwd 76 -> 79; others 64x256x14x14 -> 128
+// fwd 55 -> 40, bwd 161 -> 67; 2 x 2 16x128x16x16 -> 64 fwd 24 -> 12.
+bool packed_convT_fwd_pays(int F, int Wi, int W, int H, int R, int S, int sh, int sw) {
+    if (Wi % 4 != 0) return true;
+    if (sh == 1 && sw == 1) return F > 64;
+    return !(R == 4 && S == 4 && sh == 2 && sw == 2 && F % 32 == 0 && F <= 128 && H % 2 == 0 && W % 8 == 0);
+}
+
+bool packed_convT_bwd_pays(int F, int Wi, int C, int W, int R, int S, int sh, int sw, int ph, int pw) {
+    return Wi % 4 != 0 || W % 4 != 0 ||
+           !(R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && (C == 32 || C == 64) && F <= 192);
+}
+
 int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H, int W, int F,
                  int R, int S, int sh, int sw, int ph, int pw, const ConvEpi& epi,
                  hipStream_t st) {
@@ -400,6 +470,10 @@ int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H,
         return fail(SEERA_ERR_INVALID_ARGUMENT, "conv extent exceeds int range");
     if (npix == 0 || F == 0) return SEERA_OK;
     bool used = false;
+    if (packed_fwd_pays(C, W, F, R, S, sh, sw, ph, pw)) {
+        SEERA_TRY(packed_conv_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
+        if (used) return SEERA_OK;
+    }
     SEERA_TRY(band_conv_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, st, &used, epi));
     if (used) return SEERA_OK;
     if (s2d_applies(R, S, sh, sw)) {
@@ -618,13 +692,40 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
              int pw, hipStream_t st) {
     const int Ho = (H + 2 * ph - R) / sh + 1, Wo = (W + 2 * pw - S) / sw + 1;
     if ((int64_t)B * H * W <= 0x7fffffff && (int64_t)B * Ho * Wo <= 0x7fffffff) {
-        bool fused = false;
+        bool packed = false, fused = false;
+        if (B > 0 && packed_bwd_pays(B, C, H, W, F, R, S, sh, sw, ph, pw)) {
+            SEERA_TRY(packed_conv_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st,
+                                      &packed));
+            if (packed) return SEERA_OK;
+        }
         SEERA_TRY(fused_conv_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st,
                                  &fused));
         if (fused) return SEERA_OK;
     }
     SEERA_TRY(conv_dgrad(dY, Wconv, dX, B, F, Ho, Wo, C, H, W, R, S, sh, sw, ph, pw, st));
     return conv_wgrad(dY, X, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st);
+}
+
+int convT_fwd(const float* X, const float* Wt, float* out, int B, int F, int Hi, int Wi, int C, int H,
+              int W, int R, int S, int sh, int sw, int ph, int pw, hipStream_t st) {
+    bool used = false;
+    if (B > 0 && packed_convT_fwd_pays(F, Wi, W, H, R, S, sh, sw)) {
+        SEERA_TRY(packed_convT_fwd(X, Wt, out, B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw, st, &used));
+        if (used) return SEERA_OK;
+    }
+    return conv_dgrad(X, Wt, out, B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw, st);
+}
+
+int convT_bwd(const float* dY, const float* Wt, const float* X, float* dX, float* dW, int B, int F,
+              int Hi, int Wi, int C, int H, int W, int R, int S, int sh, int sw, int ph, int pw,
+              hipStream_t st) {
+    bool used = false;
+    if (B > 0 && packed_convT_bwd_pays(F, Wi, C, W, R, S, sh, sw, ph, pw)) {
+        SEERA_TRY(packed_convT_bwd(dY, Wt, X, dX, dW, B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw, st, &used));
+        if (used) return SEERA_OK;
+    }
+    SEERA_TRY(conv_fwd(dY, Wt, dX, B, C, H, W, F, R, S, sh, sw, ph, pw, st));
+    return conv_wgrad(X, dY, dW, nullptr, B, C, H, W, F, R, S, sh, sw, ph, pw, st);
 }
 
 int conv_wgrad(const float* Y, const float* X, float* dW, float* db, int B, int C, int H, int W,

@@ -65,6 +65,14 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
              float* db, int B, int C, int H, int W, int F, int R, int S, int sh, int sw, int ph,
              int pw, hipStream_t st);
 
+// ConvTranspose2D: out [B, C, H, W] of X [B, F, Hi, Wi] and W [F, C, R, S]; and
+// dX, dW of it from dY [B, C, H, W].
+int convT_fwd(const float* X, const float* Wt, float* out, int B, int F, int Hi, int Wi, int C, int H,
+              int W, int R, int S, int sh, int sw, int ph, int pw, hipStream_t st);
+int convT_bwd(const float* dY, const float* Wt, const float* X, float* dX, float* dW, int B, int F,
+              int Hi, int Wi, int C, int H, int W, int R, int S, int sh, int sw, int ph, int pw,
+              hipStream_t st);
+
 // ---- tensor_ops.hip: the reference's element-wise, activation, softmax,
 // broadcast, unpooling and reduction functions ----
 enum {

@@ -35,6 +35,9 @@ MUST_SEE = [
     "phase2_conv_kernel",
     "stride2_conv_kernel",
     "wgrad_s2_kernel",
+    "pack_kernel",
+    "packed_conv_kernel",
+    "packed_wgrad_kernel",
 ]
 
 _NAME = re.compile(r"remark: Function Name: (\S+)")
