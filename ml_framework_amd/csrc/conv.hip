@@ -470,6 +470,8 @@ int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H,
         return fail(SEERA_ERR_INVALID_ARGUMENT, "conv extent exceeds int range");
     if (npix == 0 || F == 0) return SEERA_OK;
     bool used = false;
+    SEERA_TRY(packed_stem_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
+    if (used) return SEERA_OK;
     if (packed_fwd_pays(C, W, F, R, S, sh, sw, ph, pw)) {
         SEERA_TRY(packed_conv_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
         if (used) return SEERA_OK;
@@ -693,6 +695,10 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
     const int Ho = (H + 2 * ph - R) / sh + 1, Wo = (W + 2 * pw - S) / sw + 1;
     if ((int64_t)B * H * W <= 0x7fffffff && (int64_t)B * Ho * Wo <= 0x7fffffff) {
         bool packed = false, fused = false;
+        if (B > 0) {
+            SEERA_TRY(packed_stem_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st, &packed));
+            if (packed) return SEERA_OK;
+        }
         if (B > 0 && packed_bwd_pays(B, C, H, W, F, R, S, sh, sw, ph, pw)) {
             SEERA_TRY(packed_conv_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st,
                                       &packed));

@@ -29,4 +29,13 @@ int packed_convT_bwd(const float* dY, const float* Wt, const float* X, float* dX
                      int F, int Hi, int Wi, int C, int H, int W, int R, int S, int sh, int sw, int ph,
                      int pw, hipStream_t st, bool* used);
 
+// The first two for a first layer (stride 2, kernel 7 or 8 wide, at most 4
+// channels) in space-to-depth form.
+int packed_stem_fwd(const float* X, const float* Wt, float* Y, int B, int C, int H, int W, int F,
+                    int R, int S, int sh, int sw, int ph, int pw, const ConvEpi& epi,
+                    hipStream_t st, bool* used);
+int packed_stem_bwd(const float* dY, const float* Wt, const float* X, float* dX, float* dW, float* db,
+                    int B, int C, int H, int W, int F, int R, int S, int sh, int sw, int ph, int pw,
+                    hipStream_t st, bool* used);
+
 }  // namespace seera

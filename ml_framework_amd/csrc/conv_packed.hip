@@ -377,17 +377,25 @@ __global__ __launch_bounds__(64 * WP * WN, 1) void packed_conv_kernel(const Pack
         }
     };
 
-    floatx16 acc[TM][TN];
+    floatx16 part[TM][TN], acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; ++r) part[i][j][r] = acc[i][j][r] = 0.f;
 
     const int wn = (wave % WN) * (BN / WN), wp = (wave / WN) * (BP / WP);
     half_pipeline<TW, TX, BK / 16, Cfg::NS, Cfg::LOADS, TM, TN>(smem, Cfg::STAGE, TW::HALVES, wn, wp, 0,
-                                                                lane, nslice, acc, load, [](int) {});
+                                                                lane, nslice, part, load, [&](int s) {
+                                                                    add_part<768 / BK>(s, part, acc);
+                                                                });
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] += part[i][j][r];
     // Lane l holds channels m0 + 32 i + 8 (e / 4) + e % 4 of pixel column l % 32.
     // The bias is in registers before the first store: a load between stores
     // would wait for them.
@@ -596,29 +604,16 @@ __global__ __launch_bounds__(64 * WF * WL * KG, 1) void packed_wgrad_kernel(cons
     constexpr int GW = WF * WL, KK = BK / 16 / KG;
     const int grp = wave / GW, gw = wave % GW;
     const int wf = (gw % WF) * (BF / WF), wl = (gw / WF) * (BL / WL);
-    // The sums of every kFlush slices are added to `sum` and begun anew: one
-    // chain over all of a split's pixels rounds more than the same products in
-    // parts (64 images of 512 channels at 7 x 7: relative error 3.5e-7 in one
-    // chain, 1.5e-7 in parts, 1.2e-7 with two groups).
-    constexpr int kFlush = 8;
+    // Parts of 16 steps, 8 where one wave takes all of a slice and the direct
+    // kernels split the pixels finely (few filters). 64 images of 512 channels at
+    // 7 x 7: relative error 3.5e-7 in one chain, 1.2e-7 in parts of 16.
+    constexpr int kPart = (KG > 1 ? 16 : 8) / KK;
     floatx16 sum[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) sum[i][j] = acc[i][j];
-    auto flush = [&](int s) {
-        if (s % kFlush == kFlush - 1) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        sum[i][j][r] += acc[i][j][r];
-                        acc[i][j][r] = 0.f;
-                    }
-        }
-    };
+    auto flush = [&](int s) { add_part<kPart>(s, acc, sum); };
     half_pipeline<TY, TXx, KK, NS, LOADS, TM, TN>(smem, STAGE, TY::HALVES, wf, wl, grp * KK, lane,
                                                   nslice, acc, load, flush);
 #pragma unroll
@@ -670,9 +665,12 @@ __device__ __forceinline__ void reduce_db(const float* __restrict__ sums, int pr
     if (g == 0 && f < F) db[f] = red[tid];
 }
 
-// dW[f, c, tap] = sum over splits of part[split][f][tap * Cp + c], in split
-// order; block (f, 64 channels), the sums through LDS so that the store is
-// contiguous. Blocks from nb_w on: db.
+// dW[f, c, tap] = sum over splits of part[split][f][tap * Cp + c]: P runs of
+// splits each added in order, the runs then in order. Block: one filter, 64 / P
+// channels, all taps; the sums through LDS so that the store is contiguous.
+// Blocks from nb_w on: db. With many splits (few, small tiles) one run would be
+// a chain of memory round trips (49 splits of 64 x 32 3x3 weights: 7.2 -> 6.4 us).
+template <int P>
 __global__ __launch_bounds__(512) void packed_wgrad_reduce(const float* __restrict__ part,
                                                            float* __restrict__ dW, int F, int C,
                                                            int Cp, int RS, int nsplit,
@@ -682,30 +680,37 @@ __global__ __launch_bounds__(512) void packed_wgrad_reduce(const float* __restri
     extern __shared__ __align__(16) float red[];
     const int tid = threadIdx.x;
     if ((int)blockIdx.x >= nb_w) return reduce_db(sums, prow, Fp, F, db, blockIdx.x - nb_w, red);
-    const int ncb = (C + 63) / 64, f = blockIdx.x / ncb, c0 = (blockIdx.x % ncb) * 64;
+    constexpr int CG = 64 / P;
+    const int ncb = (C + CG - 1) / CG, f = blockIdx.x / ncb, c0 = (blockIdx.x % ncb) * CG;
     const int L = RS * Cp;
     const int64_t stride = (int64_t)F * L;
-    const int c = tid & 63;
+    const int c = tid & (CG - 1), g = (tid & 63) / CG;
+    const int per = (nsplit + P - 1) / P, z1 = min(nsplit, (g + 1) * per);
     for (int tap = tid >> 6; tap < RS; tap += 8) {
         float s = 0.f;
         if (c0 + c < C) {
             const float* src = part + (int64_t)f * L + tap * Cp + c0 + c;
-            int z = 0;
-            for (; z + 8 <= nsplit; z += 8) {
+            int z = g * per;
+            for (; z + 8 <= z1; z += 8) {
                 float v[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = src[(z + i) * stride];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) s += v[i];
             }
-            for (; z < nsplit; ++z) s += src[z * stride];
+            for (; z < z1; ++z) s += src[z * stride];
         }
-        red[c * RS + tap] = s;
+        red[(c * RS + tap) * P + g] = s;
     }
     __syncthreads();
-    const int n = min(64, C - c0) * RS;
+    const int n = min(CG, C - c0) * RS;
     float* dst = dW + ((int64_t)f * C + c0) * RS;
-    for (int i = tid; i < n; i += 512) dst[i] = red[i];
+    for (int i = tid; i < n; i += 512) {
+        float s = red[i * P];
+#pragma unroll
+        for (int k = 1; k < P; ++k) s += red[i * P + k];
+        dst[i] = s;
+    }
 }
 
 // The same for the space-to-depth form: dW[f, c, r, q] = sum over splits of
@@ -754,8 +759,9 @@ __global__ __launch_bounds__(512) void packed_wgrad_reduce_s2d(const float* __re
 struct Packed {
     int top, left, Hp, Wp, Cp;
     int CB;
-    Packed(int top_, int left_, int Hp_, int Wp_, int C)
-        : top(top_), left(left_), Hp(Hp_), Wp(Wp_), Cp((C + 31) & ~31), CB(Cp % 64 == 0 ? 64 : 32) {}
+    Packed(int top_, int left_, int Hp_, int Wp_, int C, int round = 32)
+        : top(top_), left(left_), Hp(Hp_), Wp(Wp_), Cp((C + round - 1) / round * round),
+          CB(Cp % 64 == 0 ? 64 : 32) {}
     int lcb() const { return CB == 64 ? 6 : 5; }
     int64_t plane(int B) const { return (int64_t)B * Hp * Wp * CB; }
     int64_t halves(int B) const { return (int64_t)B * Hp * Wp * Cp; }
@@ -916,7 +922,8 @@ hipError_t launch_conv_bk(const PackedConvArgs& a, hipStream_t st) {
     const int n64 = ceil_div(a.N, 64);
     const int64_t tiles = (int64_t)ceil_div(most, 64) * a.nphase * n64;  // of 64 x 64
     if (n64 == 1) {
-        if (tiles >= 1400) return launch_conv<256, 64, 4, 1, BK>(a, most, st);
+        // (256 x 64, one block per CU, ran the first layer's forward, 4 slices
+        // deep, in 42 us; 128 x 64, two per CU, in 32)
         if (tiles >= 500) return launch_conv<128, 64, 2, 2, BK>(a, most, st);
         return launch_conv<64, 64, 2, 2, BK>(a, most, st);
     }
@@ -1019,7 +1026,11 @@ struct WgradPlan {
         a.ntf = ceil_div(F, BF);
         a.ntl = ceil_div(L, BL);
         const int tiles = a.ntf * a.ntl;
-        const int want = std::max(1, std::min(256 / std::max(tiles, 1), slices / 4));
+        // The 64-filter tiles leave room for two blocks per CU: two rounds of
+        // splits where each still has 16 slices (first layer, 6272 slices: 37.8 us
+        // with 256 blocks, 28.8 with 512).
+        const int blocks = BF == 64 && (int64_t)tiles * slices >= 512 * 16 ? 512 : 256;
+        const int want = std::max(1, std::min(blocks / std::max(tiles, 1), slices / 4));
         a.sps = ceil_div(slices, want);
         a.nsplit = ceil_div(slices, a.sps);
         a.nblocks = tiles * a.nsplit;
@@ -1061,10 +1072,12 @@ struct WgradPlan {
 
 int run_reduce(const Conv& c, const WgradPlan& wg, int Cp, float* dW, const PackAct& y, float* db,
                hipStream_t st) {
-    const int nb_w = c.F * ceil_div(c.C, 64), nb_db = db ? ceil_div(c.F, 16) : 0;
+    const bool many = wg.a.nsplit >= 16;
+    const int nb_w = c.F * ceil_div(c.C, many ? 16 : 64), nb_db = db ? ceil_div(c.F, 16) : 0;
     const size_t lds = std::max<size_t>(64 * (size_t)c.R * c.S, 512) * 4;
-    hipLaunchKernelGGL(packed_wgrad_reduce, dim3((unsigned)(nb_w + nb_db)), dim3(512), lds, st, wg.a.part,
-                       dW, c.F, c.C, Cp, c.R * c.S, wg.a.nsplit, nb_w, y.sums, y.prow, wg.a.Fp, db);
+    hipLaunchKernelGGL(many ? packed_wgrad_reduce<4> : packed_wgrad_reduce<1>, dim3((unsigned)(nb_w + nb_db)),
+                       dim3(512), lds, st, wg.a.part, dW, c.F, c.C, Cp, c.R * c.S, wg.a.nsplit, nb_w, y.sums,
+                       y.prow, wg.a.Fp, db);
     SEERA_HIP_TRY(hipGetLastError());
     return SEERA_OK;
 }
@@ -1079,7 +1092,7 @@ bool sizes_ok(const Conv& c, const Packed& x, const Packed& y) {
     const int64_t wn = (int64_t)((c.F + 31) & ~31) * ((c.C + 31) & ~31) * c.R * c.S;
     return x.halves(c.B) * 2 < kMost && y.halves(c.B) * 2 < kMost && wn * 4 < kMost &&
            (int64_t)c.B * c.H * c.W < kMost && (256 / (c.H * c.W) + 2) * ximg * 4 < kMost &&
-           (256 / (c.Ho * c.Wo) + 2) * yimg * 4 < kMost && c.R * c.S <= 36 && c.sh * c.sw <= kMaxPhase &&
+           (256 / (c.Ho * c.Wo) + 2) * yimg * 4 < kMost && c.R * c.S <= 64 && c.sh * c.sw <= kMaxPhase &&
            c.sh <= kMaxPhase && c.sw <= kMaxPhase;
 }
 
@@ -1221,6 +1234,161 @@ int packed_convT_bwd(const float* dY, const float* Wt, const float* X, float* dX
     wg.input(xp, gx, c);
     SEERA_TRY(wg.run(part, st));
     SEERA_TRY(run_reduce(c, wg, gx.Cp, dW, pk.act[0], nullptr, st));
+    *used = true;
+    return SEERA_OK;
+}
+
+namespace {
+
+// A first layer in space-to-depth form (pack_s2d): kernel 7 or 8 wide and at
+// most 8 high, stride 2, at most 4 channels. As an ordinary packed layer its
+// channels would be padded to 32.
+bool stem_ok(const Conv& c) {
+    return c.C <= 4 && c.sh == 2 && c.sw == 2 && (c.S == 7 || c.S == 8) && c.R >= 2 && c.R <= 8;
+}
+
+// X in that form: [B, Ho + T - 1, Wo + 3] pixels of 16 halves.
+struct StemInput {
+    int T, H2, W2;
+    explicit StemInput(const Conv& c) : T((c.R + 1) / 2), H2(c.Ho + T - 1), W2(c.Wo + 3) {}
+    int64_t halves(int B) const { return (int64_t)B * H2 * W2 * 16; }
+};
+
+void add_stem_act(PackArgs& pk, int& block, const float* X, half_t* out, const Conv& c, const StemInput& g) {
+    PackAct& a = pk.act[pk.nact++];
+    a.in = X; a.out = out;
+    a.total = (int64_t)c.B * c.C * c.H * c.W;
+    a.B = c.B; a.C = c.C; a.H = c.H; a.W = c.W;
+    a.Hp = g.H2; a.Wp = g.W2;
+    a.ph = c.ph; a.pw = c.pw;
+    a.s2d = 1;
+    a.by_hpwp = FastDiv(g.H2 * g.W2);
+    a.by_wp = FastDiv(g.W2);
+    a.block0 = block;
+    block += (int)(((int64_t)c.B * g.H2 * g.W2 + 255) / 256);
+}
+
+void add_stem_weights(PackArgs& pk, int& block, const float* W, half_t* out, const Conv& c, bool by_f,
+                      const Packed& gy, int64_t halves) {
+    PackS2dWeights& w = pk.w2;
+    w.in = W; w.out = out;
+    w.F = c.F; w.C = c.C; w.R = c.R; w.S = c.S;
+    w.by_f = by_f;
+    w.Fp = gy.Cp; w.lfb = gy.lcb();
+    w.items = (int)(halves / 8);
+    w.block0 = block;
+    block += ceil_div(w.items, 256);
+}
+
+bool stem_sizes_ok(const Conv& c, const StemInput& g, const Packed& gy) {
+    const int64_t ximg = (int64_t)c.C * c.H * c.W, yimg = (int64_t)c.F * c.Ho * c.Wo;
+    return g.halves(c.B) * 2 < kMost && gy.halves(c.B) * 2 < kMost && (int64_t)c.F * 8192 < kMost &&
+           (int64_t)c.B * c.H * c.W < kMost && (256 / (c.H * c.W / 4 + 1) + 2) * ximg * 4 < kMost &&
+           (256 / (c.Ho * c.Wo) + 2) * yimg * 4 < kMost;
+}
+
+}  // namespace
+
+int packed_stem_fwd(const float* X, const float* Wt, float* Y, int B, int C, int H, int W, int F,
+                    int R, int S, int sh, int sw, int ph, int pw, const ConvEpi& epi,
+                    hipStream_t st, bool* used) {
+    *used = false;
+    const Conv c{B, C, H, W, F, R, S, sh, sw, ph, pw, (H + 2 * ph - R) / sh + 1, (W + 2 * pw - S) / sw + 1};
+    if (!stem_ok(c)) return SEERA_OK;
+    const StemInput g(c);
+    if (!stem_sizes_ok(c, g, Packed(0, 0, 1, 1, F))) return SEERA_OK;
+    const int64_t xn = g.halves(B), wn = (int64_t)g.T * F * 64;
+    Scratch sc;
+    sc.need<half_t>(xn);
+    sc.need<half_t>(wn);
+    bool got = false;
+    SEERA_TRY(sc.get(st, &got));
+    if (!got) return SEERA_OK;
+    half_t* xp = sc.take<half_t>(xn);
+    half_t* wp = sc.take<half_t>(wn);
+    PackArgs pk{};
+    int block = 0;
+    add_stem_weights(pk, block, Wt, wp, c, true, Packed(0, 0, 1, 1, F), wn);
+    add_stem_act(pk, block, X, xp, c, g);
+    SEERA_TRY(launch_pack(pk, block, st));
+    PackedConvArgs a{};
+    a.x = xp; a.w = wp; a.out = Y;
+    a.x_bytes = (uint32_t)(xn * 2);
+    a.pix = 16; a.ncb = 1; a.plane = 0;
+    a.Wp = g.W2; a.HpWp = g.H2 * g.W2;
+    a.N = F; a.Hout = c.Ho; a.Wout = c.Wo;
+    a.ish = 1; a.isw = 1; a.osh = 1; a.osw = 1;
+    a.nphase = 1;
+    a.ph[0] = PackedPhase{c.Ho, c.Wo, B * c.Ho * c.Wo, g.T, 1, 0, 0, 0, 0, FastDiv(c.Ho * c.Wo), FastDiv(c.Wo)};
+    a.epi = epi;
+    SEERA_TRY(run_conv(a, 64, st));
+    *used = true;
+    return SEERA_OK;
+}
+
+int packed_stem_bwd(const float* dY, const float* Wt, const float* X, float* dX, float* dW, float* db,
+                    int B, int C, int H, int W, int F, int R, int S, int sh, int sw, int ph, int pw,
+                    hipStream_t st, bool* used) {
+    *used = false;
+    const Conv c{B, C, H, W, F, R, S, sh, sw, ph, pw, (H + 2 * ph - R) / sh + 1, (W + 2 * pw - S) / sw + 1};
+    if (!stem_ok(c)) return SEERA_OK;
+    const StemInput gx(c);
+    // The 2 x 2 blocks of the padded image that hold a pixel of the image.
+    const int ni = (H - 1 + ph) / 2 + 1, nj = (W - 1 + pw) / 2 + 1;
+    const Packed gy(gx.T - 1, 3, gx.T - 1 + std::max(c.Ho, ni), 3 + std::max(c.Wo, nj), F, 64);
+    if (!stem_sizes_ok(c, gx, gy)) return SEERA_OK;
+    const int64_t xn = gx.halves(B), yn = gy.halves(B), wn = (int64_t)gx.T * 4 * 4 * C * gy.Cp;
+    WgradPlan wg(F, gx.T * 64, c.Ho, c.Wo, B);
+    int iters, prow;
+    pack_split(B, c.Ho * c.Wo, &iters, &prow);
+    const int64_t sn = db ? (int64_t)prow * gy.Cp : 0;
+    Scratch sc;
+    sc.need<half_t>(xn);
+    sc.need<half_t>(yn);
+    sc.need<half_t>(wn);
+    sc.need<float>(wg.part_floats());
+    sc.need<float>(sn);
+    bool got = false;
+    SEERA_TRY(sc.get(st, &got));
+    if (!got) return SEERA_OK;
+    half_t* xp = sc.take<half_t>(xn);
+    half_t* yp = sc.take<half_t>(yn);
+    half_t* wp = sc.take<half_t>(wn);
+    float* part = sc.take<float>(wg.part_floats());
+    float* sums = db ? sc.take<float>(sn) : nullptr;
+    PackArgs pk{};
+    int block = 0;
+    add_stem_weights(pk, block, Wt, wp, c, false, gy, wn);
+    add_act(pk, block, dY, yp, B, F, c.Ho, c.Wo, gy, sums);
+    add_stem_act(pk, block, X, xp, c, gx);
+    SEERA_TRY(launch_pack(pk, block, st));
+
+    PackedConvArgs a{};
+    a.x = yp; a.w = wp; a.out = dX;
+    a.x_bytes = (uint32_t)(yn * 2);
+    a.pix = gy.CB; a.ncb = gy.Cp / gy.CB; a.plane = (int)gy.plane(B);
+    a.Wp = gy.Wp; a.HpWp = gy.Hp * gy.Wp;
+    a.N = 4 * C; a.Hout = H; a.Wout = W;
+    a.ish = 1; a.isw = 1; a.osh = 1; a.osw = 1;
+    a.nphase = 1;
+    a.ph[0] = PackedPhase{ni, nj, B * ni * nj, gx.T, 4, 0, ph, pw, 0, FastDiv(ni * nj), FastDiv(nj)};
+    const hipError_t e = launch_conv<128, 32, 4, 1, 64, true>(a, B * ni * nj, st);
+    if (e != hipSuccess) return fail_hip(e, "packed conv launch");
+
+    wg.output(yp, gy, B);
+    wg.a.x = xp;
+    wg.a.x_bytes = (uint32_t)(xn * 2);
+    wg.a.Cp = 64; wg.a.lcb = 6; wg.a.xplane = 0;
+    wg.a.xcol = 0; wg.a.xtap = gx.W2 * 16;
+    wg.a.xpix = 16; wg.a.xrow = wg.a.xtap; wg.a.ximg = gx.H2 * wg.a.xtap;
+    wg.a.S = 1;
+    wg.a.by_cp = FastDiv(64);
+    wg.a.by_s = FastDiv(1);
+    SEERA_TRY(wg.run(part, st));
+    const int nb_w = F * gx.T, nb_db = db ? ceil_div(F, 16) : 0;
+    hipLaunchKernelGGL(packed_wgrad_reduce_s2d, dim3((unsigned)(nb_w + nb_db)), dim3(512), 0, st, part, dW, F, C,
+                       R, S, gx.T * 64, wg.a.nsplit, nb_w, sums, pk.act[0].prow, gy.Cp, db);
+    SEERA_HIP_TRY(hipGetLastError());
     *used = true;
     return SEERA_OK;
 }

@@ -214,6 +214,24 @@ __device__ __forceinline__ void half_pipeline(half_t* smem, int stage, int b_off
     }
 }
 
+// The sums of at most PARTS slices at a time: after every PARTS-th slice the
+// accumulators are added to `sum` and begun anew. A chain of fp32 additions
+// rounds in proportion to its length, so the parts keep the error of one long
+// contraction at that of the kernels which split it.
+template <int PARTS, int TM, int TN>
+__device__ __forceinline__ void add_part(int s, floatx16 (&acc)[TM][TN], floatx16 (&sum)[TM][TN]) {
+    if (s % PARTS != PARTS - 1) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                sum[i][j][r] += acc[i][j][r];
+                acc[i][j][r] = 0.f;
+            }
+}
+
 // Wave groups that split K hand their sums to group 0 through LDS: wave w of
 // group g > 0 adds into wave w of group 0, group after group in order. `lds`
 // holds 16 * TM * TN floats per thread of one group. Called by every wave.
