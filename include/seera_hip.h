@@ -92,8 +92,8 @@ int seera_hip_matmul_async(const float *A, const float *B, float *C, int M,
  * cannot allocate device memory (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc). It calls no hipMalloc / hipFree:
  * its split-K partial sums go to a fixed 8 MiB device array that the
- * library keeps on each GPU it runs on until the process ends (no shape needs
- * more than 6.3 MB of partials today; a call that would exceed 8 MiB fails
+ * library keeps on each GPU it runs on until the process ends (plans stay
+ * within it; a call that would exceed 8 MiB fails
  * with SEERA_ERR_INVALID_ARGUMENT). The first call on each device looks up
  * the array's device address (hipGetSymbolAddress): make it outside graph
  * capture; later calls need no warm-up. Every

@@ -22,11 +22,13 @@
 
 namespace seera {
 
-// The planner (plan.h) splits K only for the 64x64 tile and only when there
-// are fewer than 128 tiles, each split over at most ceil(256 / tiles) parts
-// (and more than kMaxGroupSplits: fewer run as wave groups in the block):
-// at most 382 partial tiles of 64 x 64 fp32, 6.3 MB. 8 MiB covers every shape;
-// a request above it (a future plan) fails cleanly in workspace().
+// The planner (plan.h) splits K for the 64x64 tile when there are fewer than
+// 128 tiles, each over at most ceil(256 / tiles) parts (and more than
+// kMaxGroupSplits: fewer run as wave groups in the block): at most 382 partial
+// tiles of 64 x 64 fp32, 6.3 MB; and for the 128x128 tile as long as the
+// partials fit kNarrowPartials, this array's size (the forward's limit for
+// every entry point, so that this one gives the others' bits). 8 MiB covers
+// every shape; a request above it (a future plan) fails cleanly in workspace().
 constexpr size_t kNoAllocScratchBytes = (size_t)8 << 20;
 
 static __device__ __align__(256) float scratch[kNoAllocScratchBytes / sizeof(float)];

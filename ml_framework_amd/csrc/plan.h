@@ -25,6 +25,7 @@ struct Plan {
     int splits;
     int k_split;
     int groups = 1;  // wave groups over the K range of a 64x64 (1, 2) or 32x32 (1 .. 8) block
+    bool wide_split = false;  // split 128x128 tiles: run_plan replans where the partials' scratch is not to be had
 };
 
 constexpr int kNumCUs = 256;
@@ -59,12 +60,31 @@ inline int64_t tile_count(Tile t, int M, int N) {
     return (int64_t)((M + tile_bm(t) - 1) / tile_bm(t)) * ((N + tile_bn(t) - 1) / tile_bn(t));
 }
 
+// Partial sums that a plan may ask scratch for: kNarrowPartials where a call
+// must run in the 8 MiB of seera_hip_matmul_noalloc.
+constexpr int64_t kNarrowPartials = (int64_t)8 << 20, kWidePartials = (int64_t)64 << 20;
+
+// us of a K-long 64x64 plan (two wave groups) and of 128x128 tiles split over
+// K with their reduce, when all blocks run in one round of the CUs: 64x64 tiles
+// stream twice the operand bytes per product and took 6.1 us per 1024 of K on
+// 64 CUs and 9.6 on all (512x512x8192, both operands MN-contiguous: 49.7 us;
+// 1024x1024x8192: 79), 128x128 ones 1 us per 64-deep slice (2048^3: 31 us); the
+// reduce is a dependent launch and one pass over the partials. dB of 16x512
+// rows through a 512x512 weight 49.7 -> 25 us, of 16x1024 rows 120 -> 40.
+inline double narrow_us(int K, int64_t tiles) {
+    return 1.5 + 6.0e-3 * K * (1.0 + 0.6 * (double)std::max<int64_t>(tiles - 64, 0) / 192.0);
+}
+inline double wide_us(int ks, int64_t partial_bytes) {
+    return 3.0 + ks / 64.0 + 4.5 + (double)partial_bytes / 2.0e6;
+}
+
 // Padded work per CU (rounds of a full chip x tile area), weighted by how
 // efficiently each tile shape feeds the matrix cores; lowest wins. The 64x256
 // tile weighs a little more than 128x128: per K slice it stages 320 operand
 // rows against 256, and on equal padded work (2048^3) 128x128 ran 13% faster.
 inline Plan plan_tiles(int M, int N, int K, bool big_tiles, bool allow_split,
-                       bool allow_groups = false, bool allow_t = true) {
+                       bool allow_groups = false, bool allow_t = true,
+                       int64_t max_partials = kNarrowPartials) {
     Tile cands[4] = {Tile::L, Tile::W, Tile::M, Tile::S};
     const double eff[4] = {1.0, 1.25, 1.2, 1.6};
     Plan best{Tile::S, 1, std::max(K, 1)};
@@ -81,6 +101,25 @@ inline Plan plan_tiles(int M, int N, int K, bool big_tiles, bool allow_split,
         }
     }
     const int64_t tiles = tile_count(best.tile, M, N);
+    if (best.tile == Tile::S && big_tiles && allow_split && allow_groups && K % 64 == 0 && tiles <= kNumCUs) {
+        // Few tiles and a long K (the dB of a batch through a small weight):
+        // each 64x64 block would walk all of it.
+        const int64_t mt = tile_count(Tile::M, M, N);
+        const int want = (int)std::min<int64_t>(std::min<int64_t>(kNumCUs / mt, K / 256),
+                                                max_partials / std::max<int64_t>((int64_t)M * N * 4, 1));
+        if (want > 1) {
+            const int ks = ((K + want - 1) / want + 63) / 64 * 64, n = (K + ks - 1) / ks;
+            const int64_t bytes = (int64_t)n * M * N * 4;
+            const int s_splits = tiles < kNumCUs / 2 ? (int)std::min<int64_t>((kNumCUs + tiles - 1) / tiles, K / 128) : 1;
+            const double now = s_splits > kMaxGroupSplits ? narrow_us(K / s_splits, kNumCUs) + 5.0
+                                                          : narrow_us(K, tiles);
+            if (n > 1 && bytes <= max_partials && wide_us(ks, bytes) < 0.9 * now) {
+                Plan p{Tile::M, n, ks};
+                p.wide_split = true;
+                return p;
+            }
+        }
+    }
     if (allow_split && tiles < kNumCUs / 2 && K >= 8 * kBK) {
         int want = (int)std::min<int64_t>((kNumCUs + tiles - 1) / tiles, K / (4 * kBK));
         want = std::max(want, 1);
@@ -272,7 +311,13 @@ int run_plan(P p, const Plan& pl, hipStream_t st) {
         const size_t cn = (size_t)pl.splits * p.M * p.N;
         const size_t csn = has_colsum<P>::value ? (size_t)pl.splits * p.N : 0;
         void* ws = nullptr;
-        SEERA_TRY(workspace(sizeof(float) * (cn + csn), &ws, st));
+        if (pl.wide_split) {
+            bool got = false;
+            SEERA_TRY(workspace_try(sizeof(float) * (cn + csn), &ws, st, &got));
+            if (!got) return run_plan<BIG>(p, plan_tiles(p.M, p.N, p.K, BIG, true, pipe_ok<P>::value, true, 0), st);
+        } else {
+            SEERA_TRY(workspace(sizeof(float) * (cn + csn), &ws, st));
+        }
         p.C = static_cast<float*>(ws);
         p.ldc = p.N;
         p.split_stride = (int64_t)p.M * p.N;
@@ -326,8 +371,8 @@ inline bool pair_fits(const Plan& pl1, int M1, int N1, const Plan& pl2, int M2, 
 // tiles (one launch costs less than the smaller tile saves); returns whether
 // the plans pair, and leaves each GEMM's own best plan when they do not.
 inline bool pair_plans(int M1, int N1, int K1, int M2, int N2, int K2, Plan& pl1, Plan& pl2) {
-    pl1 = plan_tiles(M1, N1, K1, true, true, true);
-    pl2 = plan_tiles(M2, N2, K2, true, true, true);
+    pl1 = plan_tiles(M1, N1, K1, true, true, true, true, kWidePartials);
+    pl2 = plan_tiles(M2, N2, K2, true, true, true, true, kWidePartials);
     if (pair_fits(pl1, M1, N1, pl2, M2, N2)) return true;
     if (pl1.tile != Tile::T && pl2.tile != Tile::T) return false;
     const Plan q1 = plan_tiles(M1, N1, K1, true, true, true, false);

@@ -132,17 +132,15 @@ int staging_workspace(size_t bytes, void** out, hipStream_t st) {
     return pool_get(g_stage_pool, bytes, out, st);
 }
 
-int staging_workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
-    *out = nullptr;
-    *got = false;
-    if (g_fixed_owner) return SEERA_OK;
+namespace {
+int pool_try(WorkspacePool<HipBackend>& pool, size_t bytes, void** out, hipStream_t st, bool* got) {
     int dev = 0;
     SEERA_HIP_TRY(hipGetDevice(&dev));
     const bool cap = stream_capturing(st);
     int e;
     {
         std::lock_guard<std::mutex> lock(g_scratch_mu);
-        e = g_stage_pool.get(dev, st, bytes, cap, out);
+        e = pool.get(dev, st, bytes, cap, out);
     }
     if (e == WorkspacePool<HipBackend>::kGrowUnderCapture) return SEERA_OK;
     if (e == SEERA_ERR_OUT_OF_MEMORY) {
@@ -154,6 +152,25 @@ int staging_workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
     if (e != SEERA_OK) return e;
     *got = true;
     return SEERA_OK;
+}
+}  // namespace
+
+int staging_workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
+    *out = nullptr;
+    *got = false;
+    if (g_fixed_owner) return SEERA_OK;
+    return pool_try(g_stage_pool, bytes, out, st, got);
+}
+
+int workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
+    *out = nullptr;
+    *got = false;
+    if (g_fixed_owner) {
+        *got = bytes <= g_fixed_bytes;
+        if (*got) *out = g_fixed_ptr;
+        return SEERA_OK;
+    }
+    return pool_try(g_pool, bytes, out, st, got);
 }
 
 int workspace(size_t bytes, void** out, hipStream_t st) {

@@ -35,6 +35,11 @@ void clear_error();
 // (a replay still writes to it) until the device's last graph is destroyed.
 // Growing while `st` is being captured fails with SEERA_ERR_INVALID_ARGUMENT.
 int workspace(size_t bytes, void** out, hipStream_t st);
+// The same, for scratch the caller can do without: where the buffer cannot be
+// had without allocating under graph capture, the fixed workspace is too small
+// or the device is out of memory, returns SEERA_OK with *got false and nothing
+// reported.
+int workspace_try(size_t bytes, void** out, hipStream_t st, bool* got);
 // A second buffer per (device, stream) under the same rules, for operands
 // staged in a new layout before a call that itself takes workspace() (the two
 // never alias). Not available under FixedWorkspace.
