@@ -10,6 +10,7 @@
 //                           from A; split-K with a deterministic reduce
 // No transposed copies and no host loop.
 #include <algorithm>
+#include <cmath>
 
 #include "kernels.h"
 #include "plan.h"
@@ -207,34 +208,6 @@ __global__ void fill_zero_2d(float* __restrict__ C, int M, int N, int64_t ldc) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// out [rows_out, ld_out] = in [rows_in, cols_in] (leading dimension ld_in),
-// zero past its rows and columns; ld_out % 4 == 0 (one float4 store per thread).
-__global__ __launch_bounds__(256) void pad_2d(const float* __restrict__ in, int64_t ld_in,
-                                              int rows_in, int cols_in, float* __restrict__ out,
-                                              int rows_out, int ld_out) {
-    const int nq = ld_out / 4;
-    const int64_t n = (int64_t)rows_out * nq;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = i / nq;
-        const int c0 = (int)(i - r * nq) * 4;
-        floatx4 v = {0.f, 0.f, 0.f, 0.f};
-        if (r < rows_in) {
-            const float* src = in + r * ld_in;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (c0 + j < cols_in) v[j] = src[c0 + j];
-        }
-        *reinterpret_cast<floatx4*>(out + r * ld_out + c0) = v;
-    }
-}
-
-// GEMMs of at least this many multiply-adds whose operands are not
-// vector-aligned (or whose K is not a whole number of 32-deep slices) run on
-// zero-padded copies of both operands: two copy passes cost less than the
-// scalar loads (4095^3: 1.8 ms on scalar loads) or the non-streaming kernel.
-constexpr double kPadMinMacs = 4294967296.0;
-
 // Dispatch on operand vector-load eligibility. Only the 64x64 tile carries the
 // scalar (any shape / alignment) variants.
 // Optional fused forward epilogue of gemm_dispatch<..., true>.
@@ -247,7 +220,7 @@ struct Epi {
 template <bool A_KC, bool B_KC, bool EPI = false, bool COLSUM = false>
 int gemm_dispatch(const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                   int64_t ldc, int M, int N, int K, hipStream_t st, Epi epi = Epi{},
-                  float* colsum = nullptr, bool padded = false) {
+                  float* colsum = nullptr) {
     if (M == 0 || N == 0) return SEERA_OK;
     if (K == 0) {
         // Empty contraction: C = 0 (the reference's K loop never runs), then
@@ -276,41 +249,8 @@ int gemm_dispatch(const float* A, int64_t lda, const float* B, int64_t ldb, floa
         return fail(SEERA_ERR_INVALID_ARGUMENT,
                     "GEMM leading dimension too large for 32-bit tile offsets (lda=%lld ldb=%lld)",
                     (long long)lda, (long long)ldb);
-    // (padded: the staging copies below, whose rows run on in zeros or in
-    // rows that are never stored up to a multiple of 4, so that every float4
-    // load stays inside the copy)
-    const bool va = padded || (aligned16(A) && lda % 4 == 0 && (A_KC ? K : M) % 4 == 0);
-    const bool vb = padded || (aligned16(B) && ldb % 4 == 0 && (B_KC ? K : N) % 4 == 0);
-    if (!padded && (!va || !vb || K % 32 != 0) && (double)M * N * K >= kPadMinMacs) {
-        // Both operands into a staging copy: K-contiguous [rows][K32], or
-        // MN-contiguous [K32][rows rounded up to 4], zeros past the data.
-        // The zero k slices add nothing (and nothing to the column sums).
-        const int K32 = (K + 31) & ~31, M4 = (M + 3) & ~3, N4 = (N + 3) & ~3;
-        const int64_t na = A_KC ? (int64_t)M * K32 : (int64_t)K32 * M4;
-        const int64_t nb = B_KC ? (int64_t)N * K32 : (int64_t)K32 * N4;
-        const int64_t na_al = (na + 63) & ~(int64_t)63;
-        void* ws = nullptr;
-        bool got = false;
-        SEERA_TRY(staging_workspace_try(sizeof(float) * (size_t)(na_al + nb), &ws, st, &got));
-        if (got) {
-            float* Ap = static_cast<float*>(ws);
-            float* Bp = Ap + na_al;
-            auto pad = [&](const float* in, int64_t ld_in, int rows_in, int cols_in, float* out,
-                           int rows_out, int ld_out) {
-                const int64_t q = (int64_t)rows_out * (ld_out / 4);
-                const unsigned blocks = (unsigned)std::min<int64_t>((q + 255) / 256, 8192);
-                hipLaunchKernelGGL(pad_2d, dim3(blocks), dim3(256), 0, st, in, ld_in, rows_in, cols_in,
-                                   out, rows_out, ld_out);
-            };
-            if (A_KC) pad(A, lda, M, K, Ap, M, K32);
-            else pad(A, lda, K, M, Ap, K32, M4);
-            if (B_KC) pad(B, ldb, N, K, Bp, N, K32);
-            else pad(B, ldb, K, N, Bp, K32, N4);
-            SEERA_HIP_TRY(hipGetLastError());
-            return gemm_dispatch<A_KC, B_KC, EPI, COLSUM>(Ap, A_KC ? K32 : M4, Bp, B_KC ? K32 : N4, C,
-                                                          ldc, M, N, K32, st, epi, colsum, true);
-        }
-    }
+    const bool va = aligned16(A) && lda % 4 == 0 && (A_KC ? K : M) % 4 == 0;
+    const bool vb = aligned16(B) && ldb % 4 == 0 && (B_KC ? K : N) % 4 == 0;
     const Plan pl = plan_tiles(M, N, K, va && vb && big_ok, true, true);
     auto fill = [&](auto prob) {
         prob.A = A; prob.B = B; prob.C = C;
@@ -476,12 +416,67 @@ __global__ __launch_bounds__(256) void transpose_tiles4(const float* __restrict_
     }
 }
 
+// The share of the chip's 256 CUs that have work over the rounds of 256x256
+// tiles of an M x N result.
+double tile_fill(int M, int N) {
+    const double t = (double)((M + 255) / 256) * ((N + 255) / 256);
+    return t / (256.0 * std::ceil(t / 256.0));
+}
+
+// Whether an M x N product with float4-aligned rows that reads its operands
+// `reuse` times over is better off packed (below): the 256x256 tiles of the
+// streaming kernel leave CUs idle in their last round.
+bool tiles_leave_idle(int M, int N, double reuse) {
+    const double fill = tile_fill(M, N);
+    return (int64_t)((M + 255) / 256) * ((N + 255) / 256) > 256 ? fill < 0.8 && reuse >= 600
+                                                                : fill < 0.6 && reuse >= 1250;
+}
+
+// Whether a call runs on operands packed to fp16 (gemm_packed.hip). Reuse: the
+// multiply-adds per value packed. Measured without -> with (us, M x N x K; dA and dB in brackets):
+//  - rows that are not whole float4s, from kPackMin* multiply-adds on: below,
+//    the packing launch costs what it saves (332 x 539 x 103: 7.2 -> 8.8; 65 x
+//    4000 x 65 [15.4 -> 16.5]), and from a reuse of 12 [80] on (3 x 100001 x 101:
+//    18 -> 22; 16 x 4001 x 4001: 36 -> 29; 33 x 9001 x 2001: 54 -> 34 [reuse 65,
+//    76 -> 81]; 85 x 3687 x 2236 [reuse 160, 171 -> 34]); 511^3: 15.6 -> 9.7 [23.9 ->
+//    15.0], 3001 x 2047 x 1501: 60 -> 38 [141 -> 79], 4095^3: 190 -> 175 [378 -> 335].
+//  - a contraction that is not whole 32-deep slices, where the kernel cannot
+//    stream: with a reuse of 600 on (1000^3, reuse 500: 13.2 -> 14.8 [reuse 667,
+//    26.8 -> 25.1]; 1200^3: 22 -> 18 [46 -> 29]; 16384 x 512 x 500: 27 -> 32;
+//    100000 x 256 x 252: 63 -> 80 [reuse 253, 133 -> 191]).
+//  - tiles_leave_idle: 2560^3: 65 -> 54 [141 -> 105], 4608^3: 338 -> 240, 6144^3:
+//    759 -> 515 [1884 -> 995]; not 4096^3 (144 -> 167), 3584^3 (125 -> 131) or
+//    4096 x 11008 x 4096 (412 -> 438), whose tiles fill their rounds.
+constexpr double kPackMinFwd = 3e7, kPackMinBwd = 2e7;
+
+bool packed_fwd_pays(const void* A, const void* B, int M, int N, int K) {
+    const double macs = (double)M * N * K;
+    if (macs < kPackMinFwd) return false;
+    const double reuse = 1.0 / (1.0 / M + 1.0 / N);
+    if (K % 4 != 0 || N % 4 != 0 || !aligned16(A) || !aligned16(B)) return reuse >= 12;
+    if (K % 32 != 0) return reuse >= 600;
+    return tiles_leave_idle(M, N, reuse);
+}
+
+bool packed_bwd_pays(const void* A, const void* B, const void* dC, int M, int N, int K) {
+    const double macs = (double)M * N * K;
+    if (macs < kPackMinBwd) return false;
+    const double reuse = 2.0 / (1.0 / M + 1.0 / N + 1.0 / K);
+    if (K % 4 != 0 || N % 4 != 0 || !aligned16(A) || !aligned16(B) || !aligned16(dC)) return reuse >= 80;
+    if (M % 32 != 0 || N % 32 != 0) return reuse >= 600;
+    return tiles_leave_idle(M, K, reuse) || tiles_leave_idle(K, N, reuse);
+}
+
 }  // namespace
 
 int gemm_fwd(const float* A, const float* B, float* C, int M, int N, int K, int Nbatch,
              hipStream_t st) {
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
+    bool used = false;
+    if (packed_fwd_pays(A, B, (int)Mb, N, K))
+        SEERA_TRY(packed_gemm_fwd(A, B, nullptr, C, nullptr, (int)Mb, N, K, kActNone, false, st, &used));
+    if (used) return SEERA_OK;
     // A [Mb, K] row-major (K-contiguous), B [K, N] row-major (N-contiguous).
     return gemm_dispatch<true, false>(A, K, B, N, C, N, (int)Mb, N, K, st);
 }
@@ -490,6 +485,10 @@ int gemm_fwd_bias_act(const float* A, const float* B, const float* bias, float* 
                       int M, int N, int K, int Nbatch, int act, hipStream_t st) {
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
+    bool used = false;
+    if (packed_fwd_pays(A, B, (int)Mb, N, K))
+        SEERA_TRY(packed_gemm_fwd(A, B, bias, C, mask, (int)Mb, N, K, act, true, st, &used));
+    if (used) return SEERA_OK;
     Epi e;
     e.bias = bias;
     e.mask = mask;
@@ -501,6 +500,10 @@ int gemm_bwd_relu(const float* A, const float* B, const float* dC, const float* 
                   float* dB, int M, int N, int K, int Nbatch, hipStream_t st) {
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
+    bool used = false;
+    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+        SEERA_TRY(packed_gemm_bwd(A, B, dC, mask, dA, dB, nullptr, (int)Mb, N, K, st, &used));
+    if (used) return SEERA_OK;
     Epi e;
     e.mask = const_cast<float*>(mask);  // read, not written, under kActReluGrad
     e.act = kActReluGrad;
@@ -543,6 +546,10 @@ int gemm_bwd(const float* A, const float* B, const float* dC, float* dA, float* 
              int N, int K, int Nbatch, hipStream_t st) {
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
+    bool used = false;
+    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+        SEERA_TRY(packed_gemm_bwd(A, B, dC, nullptr, dA, dB, nullptr, (int)Mb, N, K, st, &used));
+    if (used) return SEERA_OK;
     // dA [Mb, K] = dC [Mb, N] . B^T : B^T element (k, n) = B[k*N + n] is
     // K-contiguous in the GEMM's contraction index n.
     // dB [K, N] = A^T [K, Mb] . dC [Mb, N]: A^T element (k, m) = A[m*K + k]
@@ -556,6 +563,10 @@ int gemm_bwd_bias(const float* A, const float* B, const float* dC, const float* 
                   float* dB, float* db, int M, int N, int K, int Nbatch, hipStream_t st) {
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
+    bool used = false;
+    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+        SEERA_TRY(packed_gemm_bwd(A, B, dC, mask, dA, dB, db, (int)Mb, N, K, st, &used));
+    if (used) return SEERA_OK;
     // dB [K, N] = A^T . dC with db[n] = sum_m dC[m, n] taken from the same
     // loads of dC (the blocks of dB's first row tile count them); with no dB
     // rows, or no rows of dC, db is its own pass (a sum of nothing is 0).

@@ -86,7 +86,7 @@ struct KcTile {
 // ---- MN-contiguous tile: BK rows (k) x R halves ----
 template <int R, int BK, int NT>
 struct McTile {
-    static_assert(R == 64 || R == 128, "rows of 128 or 256 bytes");
+    static_assert(R == 64 || R == 128 || R == 256, "rows of 128, 256 or 512 bytes");
     static constexpr int HALVES = R * BK;
     static constexpr int ITEMS = R * BK / 8;
     static constexpr int PASSES = ITEMS / NT;
@@ -96,7 +96,7 @@ struct McTile {
     // 64-byte groups of 4 consecutive rows go to different places modulo the
     // 256 bytes that one access covers.
     static __device__ __forceinline__ int swz(int k) {
-        return R == 128 ? (k & 3) << 2 : ((k >> 1) & 1) << 2;
+        return R >= 128 ? (k & 3) << 2 : ((k >> 1) & 1) << 2;
     }
     static __device__ __forceinline__ void item(int i, int& k, int& chunk) {
         k = i / CPR;

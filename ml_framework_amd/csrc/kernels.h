@@ -13,6 +13,13 @@ int gemm_fwd(const float* A, const float* B, float* C, int M, int N, int K, int 
 // writes mask = pre-activation > 0 when mask is non-null).
 int gemm_fwd_bias_act(const float* A, const float* B, const float* bias, float* C, float* mask,
                       int M, int N, int K, int Nbatch, int act, hipStream_t st);
+// The forward (bias and act as above when epi) and the backward (mask and db may
+// be null) over operands packed to fp16 (gemm_packed.hip); *used reports whether
+// they ran (false: sizes out of their range, or no staging memory).
+int packed_gemm_fwd(const float* A, const float* B, const float* bias, float* C, float* mask, int M, int N, int K,
+                    int act, bool epi, hipStream_t st, bool* used);
+int packed_gemm_bwd(const float* A, const float* B, const float* dC, const float* mask, float* dA, float* dB,
+                    float* db, int M, int N, int K, hipStream_t st, bool* used);
 // db[n] = sum_r dY[r, n] for dY [rows, N].
 int bias_grad(const float* dY, float* db, int rows, int N, hipStream_t st);
 // dA = dC . B^T, dB = A^T . dC over the folded batch.

@@ -82,6 +82,15 @@ __device__ __forceinline__ float buf_load1(rsrc_t r, uint32_t byte_off) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 0));
 }
 
+__device__ __forceinline__ float buf_load1s(rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+}
+
+// (a lane with voff >= kBufOOB stores nothing)
+__device__ __forceinline__ void buf_store1s(rsrc_t r, uint32_t voff, uint32_t soff, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, soff, 0);
+}
+
 // ---------------------------------------------------------------------------
 // LDS tile addressing.
 // ---------------------------------------------------------------------------

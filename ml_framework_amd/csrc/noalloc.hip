@@ -29,6 +29,9 @@ namespace seera {
 // partials fit kNarrowPartials, this array's size (the forward's limit for
 // every entry point, so that this one gives the others' bits). 8 MiB covers
 // every shape; a request above it (a future plan) fails cleanly in workspace().
+// There is no room here for operands packed to fp16 (gemm_packed.hip): a call
+// that runs on those elsewhere runs here on the tiles of igemm.h, whose sums
+// take another order.
 constexpr size_t kNoAllocScratchBytes = (size_t)8 << 20;
 
 static __device__ __align__(256) float scratch[kNoAllocScratchBytes / sizeof(float)];
