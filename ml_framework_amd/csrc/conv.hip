@@ -16,6 +16,7 @@
 //            = convT dW    (upsampling.cu:202-301, 354-374; roles of X, dY swapped)
 #include "conv_band.h"
 #include "conv_packed.h"
+#include "conv_pointwise.h"
 #include "gather.h"
 #include "kernels.h"
 #include "plan.h"
@@ -446,6 +447,28 @@ bool packed_bwd_pays(int B, int C, int H, int W, int F, int R, int S, int sh, in
     return C >= 128 && F >= 128;
 }
 
+// 1x1 stride-1 layers in one pass over fp32 memory (conv_pointwise.hip), which
+// takes up to 128 filters (backward 64): the blocks stream tiles of 128 pixels,
+// and a long contraction on few tiles leaves CUs without one. Measured, us, with
+// the rules below -> in one pass:
+//   fwd  64x256x56x56 -> 64 (1600 tiles)  79 -> 62    64x128x56x56 -> 96  91 -> 54
+//        64x64x56x56 -> 64   34 -> 27     32x256x28x28 -> 64 (224)  28 -> 18
+//        32x128x28x28 -> 64 (224)  11.1 -> 11.7 (not)   32x256x14x14 -> 64 (64)  12 -> 16 (not)
+//        32x64x56x56 -> 96 (800)  25 -> 26 (not)        64x192x28x28 -> 80 (448)  30 -> 27
+//   bwd  64x256x56x56 -> 64  168 -> 126   64x64x28x28 -> 32 (448)  36 -> 20
+//        16x64x28x28 -> 64 (112)  18 -> 13              64x128x28x28 -> 64 (448)  39 -> 30
+//        32x256x28x28 -> 64 (224)  32 -> 39 (not)       256x256x14x14 -> 64 (512)  59 -> 64 (not)
+int64_t pixel_tiles(int B, int H, int W) { return (int64_t)B * (((int64_t)H * W + 127) / 128); }
+
+bool pointwise_fwd_pays(int B, int C, int H, int W, int F) {
+    if (F >= 128 && (int64_t)C * F >= 128 * 128) return false;  // packed
+    const int64_t tiles = pixel_tiles(B, H, W);
+    if (F > 64) return tiles >= 1200 || (C > 128 && tiles >= 400);
+    return C <= 64 || tiles >= 800 || (C > 128 && tiles >= 200);
+}
+
+bool pointwise_bwd_pays(int B, int C, int H, int W) { return C <= 128 || pixel_tiles(B, H, W) >= 800; }
+
 // ConvTranspose2D of 4 x 4 at stride 2 keeps its direct kernels
 // (conv_phase2.hip, conv_stride2.hip) on the channel counts they take:
 // 64x128x28x28 -> 64 fwd 33 -> 55, bwd 76 -> 79; others 64x256x14x14 -> 128
@@ -472,6 +495,11 @@ int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H,
     bool used = false;
     SEERA_TRY(packed_stem_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
     if (used) return SEERA_OK;
+    const bool pointwise = R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+    if (pointwise && pointwise_fwd_pays(B, C, H, W, F)) {
+        SEERA_TRY(pointwise_conv_fwd(X, Wt, Y, B, C, (int64_t)H * W, F, epi, st, &used));
+        if (used) return SEERA_OK;
+    }
     if (packed_fwd_pays(C, W, F, R, S, sh, sw, ph, pw)) {
         SEERA_TRY(packed_conv_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
         if (used) return SEERA_OK;
@@ -698,6 +726,10 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
         if (B > 0) {
             SEERA_TRY(packed_stem_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st, &packed));
             if (packed) return SEERA_OK;
+        }
+        if (B > 0 && R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && pointwise_bwd_pays(B, C, H, W)) {
+            SEERA_TRY(pointwise_conv_bwd(dY, Wconv, X, dX, dW, db, B, C, (int64_t)H * W, F, st, &fused));
+            if (fused) return SEERA_OK;
         }
         if (B > 0 && packed_bwd_pays(B, C, H, W, F, R, S, sh, sw, ph, pw)) {
             SEERA_TRY(packed_conv_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st,

@@ -37,6 +37,8 @@ MUST_SEE = [
     "wgrad_s2_kernel",
     "pack_kernel",
     "packed_conv_kernel",
+    "pointwise_fwd_kernel",
+    "pointwise_bwd_kernel",
     "pack_matrices",
     "packed_gemm_kernel",
     "packed_wgrad_kernel",
