@@ -512,34 +512,45 @@ int gemm_bwd_relu(const float* A, const float* B, const float* dC, const float* 
         nullptr, st);
 }
 
-// db[n] = sum over rows of dY[row, n]: fixed-order partial sums of the rows a
-// thread group owns, added in group order (bit-reproducible run to run).
-constexpr int kBgCols = 64, kBgGroups = 8;
-__global__ __launch_bounds__(kBgCols * kBgGroups) void bias_grad_kernel(
-    const float* __restrict__ dY, float* __restrict__ db, int rows, int N) {
-    __shared__ float part[kBgGroups][kBgCols];
-    const int col = threadIdx.x % kBgCols, grp = threadIdx.x / kBgCols;
-    const int n = blockIdx.x * kBgCols + col;
-    const int per = (rows + kBgGroups - 1) / kBgGroups;
-    const int r0 = grp * per, r1 = min(rows, r0 + per);
+// out[n] = sum over rows of in[row, n] (rows of ld floats), in a fixed order: 16
+// columns per block, 32 classes of rows (r mod 32) each added in order with 8
+// loads in flight, then a fixed tree. Bound by latency at the sizes of a dense
+// layer: with 64 columns and 8 groups of consecutive rows per block a group's
+// loads ran one after the other on few blocks (256 x 512: 9.7 us in 8 blocks;
+// here 3.1 in 32).
+__global__ __launch_bounds__(512) void column_sums_kernel(const float* __restrict__ in, int rows, int64_t ld, int N,
+                                                          float* __restrict__ out) {
+    __shared__ float red[512];
+    const int tid = threadIdx.x, n = blockIdx.x * 16 + (tid & 15), g = tid >> 4;
     float s = 0.f;
-    if (n < N)
-        for (int r = r0; r < r1; ++r) s += dY[(int64_t)r * N + n];
-    part[grp][col] = s;
-    __syncthreads();
-    if (grp != 0 || n >= N) return;
-    float t = part[0][col];
+    if (n < N) {
+        for (int64_t r = g; r < rows; r += 8 * 32) {
+            float v[8];
 #pragma unroll
-    for (int g = 1; g < kBgGroups; ++g) t += part[g][col];
-    db[n] = t;
+            for (int i = 0; i < 8; ++i) v[i] = r + 32 * i < rows ? in[(r + 32 * i) * ld + n] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s += v[i];
+        }
+    }
+    red[tid] = s;
+    __syncthreads();
+#pragma unroll
+    for (int h = 16; h > 0; h >>= 1) {
+        if (g < h) red[tid] += red[tid + 16 * h];
+        __syncthreads();
+    }
+    if (g == 0 && n < N) out[n] = red[tid];
+}
+
+int column_sums(const float* in, float* out, int rows, int64_t ld, int N, hipStream_t st) {
+    if (N == 0) return SEERA_OK;
+    hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((N + 15) / 16)), dim3(512), 0, st, in, rows, ld, N, out);
+    SEERA_HIP_TRY(hipGetLastError());
+    return SEERA_OK;
 }
 
 int bias_grad(const float* dY, float* db, int rows, int N, hipStream_t st) {
-    if (N == 0) return SEERA_OK;
-    hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((N + kBgCols - 1) / kBgCols)),
-                       dim3(kBgCols * kBgGroups), 0, st, dY, db, rows, N);
-    SEERA_HIP_TRY(hipGetLastError());
-    return SEERA_OK;
+    return column_sums(dY, db, rows, N, N, st);
 }
 
 int gemm_bwd(const float* A, const float* B, const float* dC, float* dA, float* dB, int M,

@@ -85,33 +85,6 @@ __global__ __launch_bounds__(256) void pack_matrices(const PackMats a) {
     }
 }
 
-// db[n] = sum over the row groups of the packing pass's sums: 16 columns a
-// block, 32 classes of row groups each added in order and then in a fixed tree.
-__global__ __launch_bounds__(512) void sum_row_groups(const float* __restrict__ sums, int groups, int ld, int N,
-                                                      float* __restrict__ db) {
-    __shared__ float red[512];
-    const int tid = threadIdx.x, n = blockIdx.x * 16 + (tid & 15), g = tid >> 4;
-    float s = 0.f;
-    if (n < N) {
-        int r = g;
-        for (; r + 7 * 32 < groups; r += 8 * 32) {
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = sums[(int64_t)(r + 32 * i) * ld + n];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s += v[i];
-        }
-        for (; r < groups; r += 32) s += sums[(int64_t)r * ld + n];
-    }
-    red[tid] = s;
-    __syncthreads();
-    for (int h = 16; h > 0; h >>= 1) {
-        if (g < h) red[tid] += red[tid + 16 * h];
-        __syncthreads();
-    }
-    if (g == 0 && n < N) db[n] = red[tid];
-}
-
 // One operand as packed; KC: contracted along its columns.
 struct HalfMat {
     const half_t* p;
@@ -447,11 +420,7 @@ int packed_gemm_bwd(const float* A, const float* B, const float* dC, const float
     else
         SEERA_TRY((run_packed<true, true, false>(hc, hb, dA, M, K, K, sa, pa, part, nullptr, nullptr, 0, st)));
     SEERA_TRY((run_packed<false, false, false>(ha, hc, dB, K, N, N, sb, pb, part, nullptr, nullptr, 0, st)));
-    if (db) {
-        hipLaunchKernelGGL(sum_row_groups, dim3((unsigned)((N + 15) / 16)), dim3(512), 0, st, sums, (int)(up64(M) / 32),
-                           (int)up64(N), N, db);
-        SEERA_HIP_TRY(hipGetLastError());
-    }
+    if (db) SEERA_TRY(column_sums(sums, db, (int)(up64(M) / 32), up64(N), N, st));
     *used = true;
     return SEERA_OK;
 }

@@ -22,6 +22,8 @@ int packed_gemm_bwd(const float* A, const float* B, const float* dC, const float
                     float* db, int M, int N, int K, hipStream_t st, bool* used);
 // db[n] = sum_r dY[r, n] for dY [rows, N].
 int bias_grad(const float* dY, float* db, int rows, int N, hipStream_t st);
+// out[n] = sum over rows of in[row * ld + n], n < N.
+int column_sums(const float* in, float* out, int rows, int64_t ld, int N, hipStream_t st);
 // dA = dC . B^T, dB = A^T . dC over the folded batch.
 int gemm_bwd(const float* A, const float* B, const float* dC, float* dA, float* dB, int M, int N,
              int K, int Nbatch, hipStream_t st);
