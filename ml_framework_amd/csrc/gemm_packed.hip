@@ -4,7 +4,7 @@
 //
 // The tiles of igemm.h load fp32 operands 16 bytes at a time and round them on
 // the way to LDS; a row length that is not a multiple of 4 leaves them scalar
-// loads (511^3: 15.6 us, here 9.3; 4095^3 over zero-padded fp32 copies of both
+// loads (511^3: 15.6 us, here 9.7; 4095^3 over zero-padded fp32 copies of both
 // operands, 8 bytes moved per value each: 190 us, here 175). Here one launch
 // writes every operand of the call once as fp16 [cols / 64][rows][64], rows and
 // columns rounded up to 64 with zeros (6 bytes moved per value); a 64-deep slice
