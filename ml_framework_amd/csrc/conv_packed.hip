@@ -26,12 +26,11 @@
 #include <type_traits>
 
 #include "half_tile.h"
+#include "packed_limits.h"
 #include "runtime.h"
 
 namespace seera {
 namespace {
-
-constexpr int kMaxPhase = 9;  // strides up to 3 x 3
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
@@ -767,11 +766,6 @@ struct Packed {
     int64_t halves(int B) const { return (int64_t)B * Hp * Wp * Cp; }
 };
 
-// A convolution [B, C, H, W] -> [B, F, Ho, Wo].
-struct Conv {
-    int B, C, H, W, F, R, S, sh, sw, ph, pw, Ho, Wo;
-};
-
 struct Axis {
     int r0, T, q, n;
 };
@@ -1082,18 +1076,8 @@ int run_reduce(const Conv& c, const WgradPlan& wg, int Cp, float* dW, const Pack
     return SEERA_OK;
 }
 
-constexpr int64_t kMost = 0x7F000000ll;
-
-// Sizes that the kernels' 32-bit offsets hold: the packed tensors, one image of
-// the fp32 ones (a tile of at most 256 pixels addresses its images together),
-// and the weights; and taps that the weights' LDS tile holds.
 bool sizes_ok(const Conv& c, const Packed& x, const Packed& y) {
-    const int64_t ximg = (int64_t)c.C * c.H * c.W, yimg = (int64_t)c.F * c.Ho * c.Wo;
-    const int64_t wn = (int64_t)((c.F + 31) & ~31) * ((c.C + 31) & ~31) * c.R * c.S;
-    return x.halves(c.B) * 2 < kMost && y.halves(c.B) * 2 < kMost && wn * 4 < kMost &&
-           (int64_t)c.B * c.H * c.W < kMost && (256 / (c.H * c.W) + 2) * ximg * 4 < kMost &&
-           (256 / (c.Ho * c.Wo) + 2) * yimg * 4 < kMost && c.R * c.S <= 64 && c.sh * c.sw <= kMaxPhase &&
-           c.sh <= kMaxPhase && c.sw <= kMaxPhase;
+    return packed_sizes_ok(c, x.halves(c.B), y.halves(c.B));
 }
 
 }  // namespace
@@ -1280,13 +1264,6 @@ void add_stem_weights(PackArgs& pk, int& block, const float* W, half_t* out, con
     block += ceil_div(w.items, 256);
 }
 
-bool stem_sizes_ok(const Conv& c, const StemInput& g, const Packed& gy) {
-    const int64_t ximg = (int64_t)c.C * c.H * c.W, yimg = (int64_t)c.F * c.Ho * c.Wo;
-    return g.halves(c.B) * 2 < kMost && gy.halves(c.B) * 2 < kMost && (int64_t)c.F * 8192 < kMost &&
-           (int64_t)c.B * c.H * c.W < kMost && (256 / (c.H * c.W / 4 + 1) + 2) * ximg * 4 < kMost &&
-           (256 / (c.Ho * c.Wo) + 2) * yimg * 4 < kMost;
-}
-
 }  // namespace
 
 int packed_stem_fwd(const float* X, const float* Wt, float* Y, int B, int C, int H, int W, int F,
@@ -1296,7 +1273,7 @@ int packed_stem_fwd(const float* X, const float* Wt, float* Y, int B, int C, int
     const Conv c{B, C, H, W, F, R, S, sh, sw, ph, pw, (H + 2 * ph - R) / sh + 1, (W + 2 * pw - S) / sw + 1};
     if (!stem_ok(c)) return SEERA_OK;
     const StemInput g(c);
-    if (!stem_sizes_ok(c, g, Packed(0, 0, 1, 1, F))) return SEERA_OK;
+    if (!stem_sizes_ok(c, g.halves(B), 0, c.Ho * (int64_t)c.Wo)) return SEERA_OK;
     const int64_t xn = g.halves(B), wn = (int64_t)g.T * F * 64;
     Scratch sc;
     sc.need<half_t>(xn);
@@ -1336,7 +1313,7 @@ int packed_stem_bwd(const float* dY, const float* Wt, const float* X, float* dX,
     // The 2 x 2 blocks of the padded image that hold a pixel of the image.
     const int ni = (H - 1 + ph) / 2 + 1, nj = (W - 1 + pw) / 2 + 1;
     const Packed gy(gx.T - 1, 3, gx.T - 1 + std::max(c.Ho, ni), 3 + std::max(c.Wo, nj), F, 64);
-    if (!stem_sizes_ok(c, gx, gy)) return SEERA_OK;
+    if (!stem_sizes_ok(c, gx.halves(B), gy.halves(B), (int64_t)ni * nj)) return SEERA_OK;
     const int64_t xn = gx.halves(B), yn = gy.halves(B), wn = (int64_t)gx.T * 4 * 4 * C * gy.Cp;
     WgradPlan wg(F, gx.T * 64, c.Ho, c.Wo, B);
     int iters, prow;
