@@ -44,10 +44,16 @@ typedef int dma_rsrc_t __attribute__((ext_vector_type(4)));
 // 43.6 against 27.2 us). The callers wait (wait_vm) before a barrier that precedes the reads.
 __device__ __forceinline__ void dma16(dma_rsrc_t r, half_t* lds, uint32_t voff, uint32_t soff) {
     const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) half_t*)lds;
+    // M0 holds the LDS address. The compiler never allocates it, and warns that a
+    // clobber of it will not be preserved, which is what is meant: an M0 that it
+    // set up itself before this statement has to be set up again after it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(at), "v"(voff), "s"(r), "s"(soff)
-                 : "memory");
+                 : "memory", "m0");
+#pragma clang diagnostic pop
 }
 
 // The words of a buffer resource over `bytes` bytes at `base` (wave-uniform; at
