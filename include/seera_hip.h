@@ -95,9 +95,9 @@ int seera_hip_matmul_async(const float *A, const float *B, float *C, int M,
  * library keeps on each GPU it runs on until the process ends (plans stay
  * within it; a call that would exceed 8 MiB fails
  * with SEERA_ERR_INVALID_ARGUMENT). Its result has seera_hip_matmul_async's
- * bits, except where that call packs its operands to fp16 in its own scratch
- * first (rows that are not whole float4s, ragged or large shapes): there only
- * the order of the fp32 sums differs. The first call on each device looks up
+ * bits, except where that call packs more than 8 MiB of operands to fp16 first
+ * (rows that are not whole float4s, ragged or large shapes): there only the
+ * order of the fp32 sums differs. The first call on each device looks up
  * the array's device address (hipGetSymbolAddress): make it outside graph
  * capture; later calls need no warm-up. Every
  * call on one GPU shares that array, so calls that overlap on one GPU (on two

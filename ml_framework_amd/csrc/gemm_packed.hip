@@ -369,7 +369,9 @@ int packed_gemm_fwd(const float* A, const float* B, const float* bias, float* C,
     const size_t np = pl.splits > 1 ? (size_t)pl.splits * M * N * 4 : 0;
     void* ws = nullptr;
     bool got = false;
-    SEERA_TRY(staging_workspace_try(na + nb + np, &ws, st, &got));
+    // (operands and partials in one piece: what fits the fixed array of the
+    // no-allocation entry point runs there in the same order of sums)
+    SEERA_TRY(staging_workspace_try(na + nb + np, &ws, st, &got, true));
     if (!got) return SEERA_OK;
     char* p = static_cast<char*>(ws);
     PackMats pk{};

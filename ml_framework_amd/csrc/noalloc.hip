@@ -2,8 +2,9 @@
 // cannot allocate device memory (code under HIP graph capture, serving
 // loops, harnesses that forbid hipMalloc).
 //
-// The only device memory the GEMM needs beyond its inputs and output is the
-// split-K partial sums (plan.h run_plan). Here they go to `scratch`, a fixed
+// The device memory the GEMM uses beyond its inputs and output is the split-K
+// partial sums (plan.h run_plan) and, for shapes that gain from it, operands
+// packed to fp16 (gemm_packed.hip). Here both go to `scratch`, a fixed
 // array of kNoAllocScratchBytes that the code object carries: the runtime
 // places one copy on each GPU the library runs on, kept until the process
 // ends. Its device address is taken once per device with hipGetSymbolAddress
@@ -11,7 +12,7 @@
 // kernels through a FixedWorkspace, exactly as the allocating entry point
 // hands them its workspace. Nothing is allocated or freed per call.
 //
-// The split-K partials of a call are written in full before they are read,
+// Partials and packed operands of a call are written in full before they are read,
 // so the array needs no clearing. Every call on a GPU shares that GPU's
 // array: calls that overlap on one GPU (queued on two streams, or from two
 // host threads) race on it.
@@ -29,8 +30,8 @@ namespace seera {
 // partials fit kNarrowPartials, this array's size (the forward's limit for
 // every entry point, so that this one gives the others' bits). 8 MiB covers
 // every shape; a request above it (a future plan) fails cleanly in workspace().
-// There is no room here for operands packed to fp16 (gemm_packed.hip): a call
-// that runs on those elsewhere runs here on the tiles of igemm.h, whose sums
+// Calls that pack their operands to fp16 (gemm_packed.hip) do so here too while
+// operands and partials fit; beyond, they run on the tiles of igemm.h, whose sums
 // take another order.
 constexpr size_t kNoAllocScratchBytes = (size_t)8 << 20;
 

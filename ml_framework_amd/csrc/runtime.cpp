@@ -155,21 +155,25 @@ int pool_try(WorkspacePool<HipBackend>& pool, size_t bytes, void** out, hipStrea
 }
 }  // namespace
 
-int staging_workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
+namespace {
+int fixed_try(size_t bytes, void** out, bool* got) {
+    *got = bytes <= g_fixed_bytes;
+    if (*got) *out = g_fixed_ptr;
+    return SEERA_OK;
+}
+}  // namespace
+
+int staging_workspace_try(size_t bytes, void** out, hipStream_t st, bool* got, bool sole) {
     *out = nullptr;
     *got = false;
-    if (g_fixed_owner) return SEERA_OK;
+    if (g_fixed_owner) return sole ? fixed_try(bytes, out, got) : SEERA_OK;
     return pool_try(g_stage_pool, bytes, out, st, got);
 }
 
 int workspace_try(size_t bytes, void** out, hipStream_t st, bool* got) {
     *out = nullptr;
     *got = false;
-    if (g_fixed_owner) {
-        *got = bytes <= g_fixed_bytes;
-        if (*got) *out = g_fixed_ptr;
-        return SEERA_OK;
-    }
+    if (g_fixed_owner) return fixed_try(bytes, out, got);
     return pool_try(g_pool, bytes, out, st, got);
 }
 

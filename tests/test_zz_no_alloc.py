@@ -88,3 +88,26 @@ def test_noalloc_argument_checks(lib):
         capi.SEERA_ERR_INVALID_ARGUMENT
     assert lib.seera_hip_matmul_noalloc(None, None, None, 2, 2, 2, 1, None) == \
         capi.SEERA_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("M,N,K,nb", [(333, 257, 515, 1), (511, 511, 511, 2), (130, 70, 4099, 1), (1023, 1023, 1023, 1),
+                                      (1300, 1300, 1300, 1), (384, 512, 8190, 1)])
+def test_noalloc_on_packed_shapes(lib, M, N, K, nb):
+    """Shapes whose operands are packed to fp16 first, split (130 x 70, 384 x 512)
+    and not: up to the array's 8 MiB the bits of seera_hip_matmul_async, beyond
+    (the last) its result in another order of the fp32 sums."""
+    st = ctypes.c_void_p()
+    capi.check(lib.seera_hip_stream_create(ctypes.byref(st)))
+    r = np.random.default_rng(M)
+    a = r.uniform(-1, 1, (nb, M, K)).astype(np.float32)
+    b = r.uniform(-1, 1, (K, N)).astype(np.float32)
+    try:
+        want = _run(lib, "seera_hip_matmul_async", a, b, M, N, K, nb, st.value)
+        got = _run(lib, "seera_hip_matmul_noalloc", a, b, M, N, K, nb, st.value)
+    finally:
+        lib.seera_hip_stream_destroy(st.value)
+    if K < 8000:
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    else:
+        # two orders of K additions, each off by at most 0.41 * 2^-24 * sqrt(K / 2)
+        assert np.linalg.norm(got - want) <= 4e-6 * np.linalg.norm(want)
