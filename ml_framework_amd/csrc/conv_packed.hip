@@ -294,7 +294,37 @@ struct PackedConvArgs {
     FastDiv by_ntn, by_phase;
     PackedPhase ph[kMaxPhase];
     ConvEpi epi;
+    int R, S;             // kS2d*: the kernel's own rows and columns
 };
+
+// What the product is of. kS2dForward, kS2dInput: a first layer in
+// space-to-depth form, whose 2 T x 8 taps are rounded up from R x S.
+enum PackedKind { kPlain, kS2dForward, kS2dInput };
+
+// One sum of a space-to-depth product over the kernel's own taps. The matrix
+// cores also multiply the added taps' zero weights, and 0 * inf is NaN where an
+// infinite operand is no term of the output: a lane that finds NaN takes the sum
+// from here. n: output channel; pi, pj: the output pixel in the phase's grid.
+template <int BK, PackedKind KIND>
+__device__ __forceinline__ float own_taps_sum(const PackedConvArgs& a, int b, int pi, int pj, int n) {
+    const PackedPhase& ph = a.ph[0];
+    const int taps = ph.T * ph.U;
+    float s = 0.f;
+    for (int cb = 0; cb < a.ncb; ++cb)
+        for (int tap = 0; tap < taps; ++tap) {
+            const int t = tap / ph.U, u = tap - t * ph.U;
+            const half_t* x = a.x + cb * (int64_t)a.plane + ph.x0 +
+                              (int64_t)(b * a.HpWp + (pi * a.ish + t) * a.Wp + pj * a.isw + u) * a.pix;
+            const half_t* w = a.w + ph.woff + ((int64_t)(cb * taps + tap) * a.N + n) * BK;
+            for (int k = 0; k < BK; ++k) {
+                // (the forward's slice is a kernel row: 4 columns of 2 x 2 x 4 channels)
+                const int c2 = KIND == kS2dForward ? k & 15 : n, col = KIND == kS2dForward ? k >> 4 : 3 - u;
+                const int row = KIND == kS2dForward ? t : ph.T - 1 - t;
+                if (2 * row + ((c2 >> 1) & 1) < a.R && 2 * col + (c2 & 1) < a.S) s += (float)x[k] * (float)w[k];
+            }
+        }
+    return s;
+}
 
 // BP pixels x BN output channels per block, WP x WN waves, three LDS stages.
 template <int BP, int BN, int WP, int WN, int BK>
@@ -307,10 +337,10 @@ struct PackedCfg {
     static constexpr int LOADS = TX::PASSES + TW::PASSES;  // DMA instructions per wave and slice
 };
 
-// D2S: the output is the space-to-depth form's dX, stored to the image it came
+// kS2dInput: the output is the space-to-depth form's dX, stored to the image it came
 // from: channel (c * 2 + dy) * 2 + dx of pixel (i, j) is pixel (2 i + dy - oph,
 // 2 j + dx - opw) of channel c (oph, opw: the padding), where that lies inside.
-template <int BP, int BN, int WP, int WN, int BK, bool D2S>
+template <int BP, int BN, int WP, int WN, int BK, PackedKind KIND>
 __global__ __launch_bounds__(64 * WP * WN, 1) void packed_conv_kernel(const PackedConvArgs a) {
     using Cfg = PackedCfg<BP, BN, WP, WN, BK>;
     using TX = typename Cfg::TX;
@@ -420,28 +450,38 @@ __global__ __launch_bounds__(64 * WP * WN, 1) void packed_conv_kernel(const Pack
     // Stores through a resource over the block's images: a lane past the phase's
     // pixels or the channels gets an offset that the hardware drops.
     const int b0 = ph.by_howo.div(q0), left = a.N - m0;
-    const int64_t img = (int64_t)(D2S ? a.N >> 2 : a.N) * plane;
+    const int64_t img = (int64_t)(KIND == kS2dInput ? a.N >> 2 : a.N) * plane;
     const rsrc_t ro = make_rsrc(a.out + b0 * img), rm = make_rsrc((mp ? mp : a.out) + b0 * img);
     const uint32_t step = (uint32_t)plane * 4u;
-    if constexpr (D2S) {
+    static_assert(TM * 16 <= 32, "one bit per sum of a column");
+    if constexpr (KIND == kS2dInput) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int q = q0 + wp + 32 * j + (lane & 31);
             const int b = ph.by_howo.div(q), r = q - b * HoWo;
             const int pi = ph.by_wo.div(r), pj = r - pi * ph.Wo;
             const int h0 = 2 * pi - ph.oph, w0 = 2 * pj - ph.opw;
+            auto put = [&](int n, float v) {
+                const int h = h0 + ((n >> 1) & 1), w = w0 + (n & 1);
+                const bool in = q < ph.npix && n < a.N && (unsigned)h < (unsigned)a.Hout &&
+                                (unsigned)w < (unsigned)a.Wout;
+                const uint32_t o = (uint32_t)((b - b0) * img + (n >> 2) * plane + h * a.Wout + w) * 4u;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ro, in ? o : kBufOOB, 0, 0);
+            };
+            uint32_t nan = 0;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const int n = m0 + chan(i, e), h = h0 + ((n >> 1) & 1), w = w0 + (n & 1);
-                    const bool in = q < ph.npix && n < a.N && (unsigned)h < (unsigned)a.Hout &&
-                                    (unsigned)w < (unsigned)a.Wout;
-                    const uint32_t o = (uint32_t)((b - b0) * img + (n >> 2) * plane + h * a.Wout + w) * 4u;
                     const float v = acc[i][j][e];
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ro,
-                                                          in ? o : kBufOOB, 0, 0);
+                    put(m0 + chan(i, e), v);
+                    nan |= v != v ? 1u << (i * 16 + e) : 0u;
                 }
+            if (q >= ph.npix) nan = 0;
+            for (; nan != 0; nan &= nan - 1) {
+                const int k = __builtin_ctz(nan), n = m0 + chan(k >> 4, k & 15);
+                if (n < a.N) put(n, own_taps_sum<BK, KIND>(a, b, pi, pj, n));
+            }
         }
         return;
     }
@@ -455,21 +495,31 @@ __global__ __launch_bounds__(64 * WP * WN, 1) void packed_conv_kernel(const Pack
                                           (int64_t)(oh * a.osh + ph.oph) * a.Wout + ow * a.osw +
                                           ph.opw) * 4u;
             const int nl = q < ph.npix ? left : 0;
+            auto put = [&](uint32_t at, uint32_t row, float v) {
+                const float y = decltype(relu)::value ? (v > 0.f ? v : 0.f) : v;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), ro, at, row, 0);
+                if (decltype(mask)::value) {
+                    const float k = v > 0.f ? 1.f : 0.f;
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, k), rm, at, row, 0);
+                }
+            };
+            uint32_t nan = 0;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const float v = acc[i][j][e];
-                    const uint32_t at = chan(i, e) < nl ? o : kBufOOB;
-                    const float y = decltype(relu)::value ? (v > 0.f ? v : 0.f) : v;
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), ro, at,
-                                                          chan(i, e) * step, 0);
-                    if (decltype(mask)::value) {
-                        const float k = v > 0.f ? 1.f : 0.f;
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, k), rm, at,
-                                                              chan(i, e) * step, 0);
-                    }
+                    put(chan(i, e) < nl ? o : kBufOOB, chan(i, e) * step, v);
+                    if constexpr (KIND == kS2dForward) nan |= v != v ? 1u << (i * 16 + e) : 0u;
                 }
+            if constexpr (KIND == kS2dForward) {
+                for (; nan != 0; nan &= nan - 1) {
+                    const int k = __builtin_ctz(nan), c = chan(k >> 4, k & 15);
+                    if (c < nl)
+                        put(o + (uint32_t)c * step, 0u,
+                            own_taps_sum<BK, KIND>(a, b, oh, ow, m0 + c) + (bp ? bp[m0 + c] : 0.f));
+                }
+            }
         }
     };
     constexpr std::true_type yes;
@@ -881,10 +931,10 @@ int launch_pack(const PackArgs& pk, int blocks, hipStream_t st) {
     return SEERA_OK;
 }
 
-template <int BP, int BN, int WP, int WN, int BK, bool D2S = false>
+template <int BP, int BN, int WP, int WN, int BK, PackedKind KIND>
 hipError_t launch_conv(PackedConvArgs a, int most, hipStream_t st) {
     using Cfg = PackedCfg<BP, BN, WP, WN, BK>;
-    auto kern = packed_conv_kernel<BP, BN, WP, WN, BK, D2S>;
+    auto kern = packed_conv_kernel<BP, BN, WP, WN, BK, KIND>;
     static_assert(Cfg::LDS_BYTES <= 160 * 1024, "LDS of one CU");
     if (Cfg::LDS_BYTES > 65536) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -908,7 +958,7 @@ hipError_t launch_conv(PackedConvArgs a, int most, hipStream_t st) {
 //   64x256x14x14     41.4     33.1     37.4    41.6
 //   64x512x7x7       58.0     40.7     38.5    37.6
 //   8x256x14x14      31.6     22.7     20.4    18.2
-template <int BK>
+template <int BK, PackedKind KIND = kPlain>
 hipError_t launch_conv_bk(const PackedConvArgs& a, hipStream_t st) {
     int most = 0;
     for (int z = 0; z < a.nphase; ++z) most = std::max(most, a.ph[z].npix);
@@ -918,13 +968,13 @@ hipError_t launch_conv_bk(const PackedConvArgs& a, hipStream_t st) {
     if (n64 == 1) {
         // (256 x 64, one block per CU, ran the first layer's forward, 4 slices
         // deep, in 42 us; 128 x 64, two per CU, in 32)
-        if (tiles >= 500) return launch_conv<128, 64, 2, 2, BK>(a, most, st);
-        return launch_conv<64, 64, 2, 2, BK>(a, most, st);
+        if (tiles >= 500) return launch_conv<128, 64, 2, 2, BK, KIND>(a, most, st);
+        return launch_conv<64, 64, 2, 2, BK, KIND>(a, most, st);
     }
-    if (tiles >= 1400) return launch_conv<256, 128, 4, 2, BK>(a, most, st);
-    if (tiles >= 600) return launch_conv<128, 128, 4, 2, BK>(a, most, st);
-    if (tiles >= 300) return launch_conv<64, 128, 2, 2, BK>(a, most, st);
-    return launch_conv<64, 64, 2, 2, BK>(a, most, st);
+    if (tiles >= 1400) return launch_conv<256, 128, 4, 2, BK, KIND>(a, most, st);
+    if (tiles >= 600) return launch_conv<128, 128, 4, 2, BK, KIND>(a, most, st);
+    if (tiles >= 300) return launch_conv<64, 128, 2, 2, BK, KIND>(a, most, st);
+    return launch_conv<64, 64, 2, 2, BK, KIND>(a, most, st);
 }
 
 int run_conv(const PackedConvArgs& a, int CB, hipStream_t st) {
@@ -1298,7 +1348,9 @@ int packed_stem_fwd(const float* X, const float* Wt, float* Y, int B, int C, int
     a.nphase = 1;
     a.ph[0] = PackedPhase{c.Ho, c.Wo, B * c.Ho * c.Wo, g.T, 1, 0, 0, 0, 0, FastDiv(c.Ho * c.Wo), FastDiv(c.Wo)};
     a.epi = epi;
-    SEERA_TRY(run_conv(a, 64, st));
+    a.R = R; a.S = S;
+    const hipError_t e = launch_conv_bk<64, kS2dForward>(a, st);
+    if (e != hipSuccess) return fail_hip(e, "packed conv launch");
     *used = true;
     return SEERA_OK;
 }
@@ -1349,7 +1401,8 @@ int packed_stem_bwd(const float* dY, const float* Wt, const float* X, float* dX,
     a.ish = 1; a.isw = 1; a.osh = 1; a.osw = 1;
     a.nphase = 1;
     a.ph[0] = PackedPhase{ni, nj, B * ni * nj, gx.T, 4, 0, ph, pw, 0, FastDiv(ni * nj), FastDiv(nj)};
-    const hipError_t e = launch_conv<128, 32, 4, 1, 64, true>(a, B * ni * nj, st);
+    a.R = R; a.S = S;
+    const hipError_t e = launch_conv<128, 32, 4, 1, 64, kS2dInput>(a, B * ni * nj, st);
     if (e != hipSuccess) return fail_hip(e, "packed conv launch");
 
     wg.output(yp, gy, B);

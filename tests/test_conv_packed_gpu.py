@@ -139,3 +139,47 @@ def test_infinities_stay_where_they_belong():
     hit[:, 3, 0:2, 1:3] = True
     hit[7] = True
     assert np.all(np.isfinite(dw[~hit]))
+
+
+@pytest.mark.parametrize("N,C,H,W,F,KH,KW,p", [(2, 3, 31, 29, 33, 7, 7, 3), (1, 4, 22, 24, 130, 7, 7, 2), (3, 1, 18, 26, 70, 5, 7, 2),
+                                               (2, 2, 24, 28, 64, 8, 8, 3), (20, 3, 64, 62, 40, 7, 7, 3)], ids=str)
+def test_first_layer_infinities_stay_where_they_belong(N, C, H, W, F, KH, KW, p):
+    """The space-to-depth form multiplies real values by the zero weights of the
+    taps that it adds: an infinite one must reach the outputs that it is a term
+    of and leave the others, rows and columns beside them included, as they are."""
+    x, w, dy = _data(f"stem{N}{F}", N, C, H, W, F, KH, KW, 2, p)
+    b = np.random.default_rng(7).standard_normal(F).astype(np.float32)
+    OH, OW = dy.shape[2:]
+    spots = [(0, 0, 0, 0), (N - 1, C - 1, H - 1, W - 1), (0, C - 1, H // 2, W // 2 + 1)]
+    hit = np.zeros(dy.shape, bool)
+    for n, c, h, v in spots:
+        x[n, c, h, v] = np.inf
+        for r in range(KH):
+            for q in range(KW):
+                i, j = h + p - r, v + p - q
+                if i % 2 == 0 and j % 2 == 0 and 0 <= i // 2 < OH and 0 <= j // 2 < OW:
+                    hit[n, :, i // 2, j // 2] = True
+    with _dev(x) as px, _dev(w) as pw, _dev(b) as pb, _out(dy.shape) as py:
+        capi.call("seera_hip_conv2d_fwd_bias_act", px.ptr, pw.ptr, pb.ptr, py.ptr, 0, N, C, H, W, F, KH, KW, p, p, 2, 2, 0)
+        y = py.to_array(dy.shape)
+    np.testing.assert_array_equal(np.isfinite(y), ~hit)
+    x[~np.isfinite(x)] = 0
+    want = S.conv2d_forward(fp16r(x), fp16r(w), 2, 2, p, p) + b[None, :, None, None]
+    assert_parity(y[~hit], want[~hit], "fwd", STRICT)
+
+    hit = np.zeros(x.shape, bool)
+    for n, f, i, j in [(0, 1, 0, 0), (N - 1, F - 1, OH - 1, OW - 1), (0, F // 2, OH // 2, OW // 2)]:
+        dy[n, f, i, j] = -np.inf
+        for r in range(KH):
+            for q in range(KW):
+                h, v = 2 * i - p + r, 2 * j - p + q
+                if 0 <= h < H and 0 <= v < W:
+                    hit[n, :, h, v] = True
+    dx, dw = hip_conv_bwd(dy, x, w, 2, p)
+    np.testing.assert_array_equal(np.isfinite(dx), ~hit)
+    bad = ~np.isfinite(dy).all((0, 2, 3))
+    assert np.isfinite(dw[~bad]).all()
+    dy[~np.isfinite(dy)] = 0
+    rdx, rdw = S.conv2d_backward(fp16r(dy), fp16r(x), fp16r(w), 2, 2, p, p)
+    assert_parity(dx[~hit], rdx[~hit], "dX", STRICT)
+    assert_parity(dw[~bad], rdw[~bad], "dW", STRICT)
