@@ -15,9 +15,13 @@ from tests.helpers import _dev, _out, assert_parity, hip_conv_bwd, hip_conv_fwd,
 
 pytestmark = pytest.mark.gpu
 S = oracle.seera_cpp
-# fp32 sums of the same fp16 products in another order: 2^-24 per addition,
-# growing with the square root of the number of terms (at most 50 thousand
-# here, in dW): 2^-24 * 220 = 1.3e-5 at the very worst, 1e-6 seen.
+# fp32 sums of the same fp16 products in another order. Each addition rounds the
+# partial sum by 0.41 * 2^-24 of it (root mean square); over a chain of n terms of
+# random sign the partial sums grow with the square root of their length, so the
+# result is off by about 0.41 * 2^-24 * sqrt(n / 2): 3.9e-6 at the 50 thousand
+# terms of the longest dW here. The oracle's chain may be off as much: 5.5e-6
+# together, stated with less than a factor of two. (A term lost or read twice
+# shows in test_exact.)
 STRICT = 1e-5
 
 
@@ -52,9 +56,23 @@ CASES = [
     ("stem_5x7", 2, 3, 17, 20, 40, 5, 7, 2, 2),
     ("stem_tiles", 6, 3, 112, 112, 64, 7, 7, 2, 3),
     ("rows_1xk", 2, 36, 4, 30, 36, 1, 7, 1, 3),
-    ("tiles_128", 20, 32, 30, 30, 128, 3, 3, 1, 1),   # 128 x 128 tiles
-    ("tiles_256", 25, 32, 31, 31, 200, 3, 3, 1, 1),   # 256 x 128 tiles, 256 x 64 for dX
-    ("dw_splits", 40, 64, 30, 30, 64, 3, 3, 1, 1),    # 64 x 128 dW tiles, many splits
+    ("tiles_128", 20, 32, 30, 30, 128, 3, 3, 1, 1),   # 64 x 128 tiles in 32-deep slices
+    ("tiles_256", 25, 32, 31, 31, 200, 3, 3, 1, 1),   # 256 x 128 tiles in 32-deep slices
+    ("dw_splits", 40, 64, 30, 30, 64, 3, 3, 1, 1),    # 128 x 64 tiles; 64 x 128 dW tiles, many splits
+]
+
+# Every tile (pixels x channels) in 64- and 32-deep slices, forward and dX, with
+# pixels and channels that are no multiple of it.
+TILE_CASES = [
+    ("bk64_64x128", 8, 190, 29, 31, 190, 3, 3, 1, 1),
+    ("bk64_128x128", 17, 190, 29, 31, 190, 3, 3, 1, 1),
+    ("bk64_256x128", 34, 190, 29, 31, 190, 2, 2, 1, 1),
+    ("bk32_64x128", 8, 150, 29, 31, 150, 3, 3, 1, 1),
+    ("bk32_128x128", 17, 150, 29, 31, 150, 3, 3, 1, 1),
+    ("bk32_256x128", 34, 150, 29, 31, 150, 2, 2, 1, 1),
+    ("s2_256x128", 33, 130, 29, 31, 64, 3, 3, 2, 1),   # dX in four residues of 15 x 16 to 14 x 15
+    ("bk64_128x64", 37, 60, 29, 31, 62, 3, 3, 1, 1),
+    ("bk32_128x64", 37, 30, 29, 31, 28, 3, 3, 1, 1),
 ]
 
 
@@ -76,6 +94,31 @@ def test_conv2d(case):
     rdx, rdw = S.conv2d_backward(fp16r(dy), fp16r(x), fp16r(w), s, s, p, p)
     assert_parity(dx, rdx, name + " dX", STRICT)
     assert_parity(dw, rdw, name + " dW", STRICT, mabs=2e-2 * max(1.0, float(np.abs(rdw).max()) / 100))
+
+
+@pytest.mark.parametrize("case", CASES + TILE_CASES, ids=[c[0] for c in CASES + TILE_CASES])
+def test_exact(case):
+    """Small whole numbers: every product and partial sum (below 2^24) is exact
+    in fp16 and fp32, so the results are the oracle's bits."""
+    name, N, C, H, W, F, KH, KW, s, p = case
+    r = np.random.default_rng(zlib.crc32(name.encode()))
+    OH, OW = out_hw(H, W, KH, KW, s, p)
+    x, w, dy, b = (r.integers(-2, 3, sh).astype(np.float32) for sh in ((N, C, H, W), (F, C, KH, KW), (N, F, OH, OW), (F,)))
+    y = S.conv2d_forward(x, w, s, s, p, p)
+    np.testing.assert_array_equal(hip_conv_fwd(x, w, s, p), y)
+    rdx, rdw = S.conv2d_backward(dy, x, w, s, s, p, p)
+    with _dev(x) as px, _dev(w) as pw, _dev(b) as pb, _dev(dy) as pdy, _out(dy.shape) as py, _out(dy.shape) as pm, \
+            _out(x.shape) as pdx, _out(w.shape) as pdw, _out((F,)) as pdb:
+        capi.call("seera_hip_conv2d_fwd_bias_act", px.ptr, pw.ptr, pb.ptr, py.ptr, pm.ptr, N, C, H, W, F, KH, KW,
+                  p, p, s, s, capi.SEERA_ACT_RELU)
+        capi.call("seera_hip_conv2d_bwd_bias", pw.ptr, px.ptr, pdy.ptr, pdx.ptr, pdw.ptr, pdb.ptr, N, C, H, W, F,
+                  KH, KW, s, s, p, p)
+        y += b[None, :, None, None]
+        np.testing.assert_array_equal(py.to_array(y.shape), np.maximum(y, 0))
+        np.testing.assert_array_equal(pm.to_array(y.shape), (y > 0).astype(np.float32))
+        np.testing.assert_array_equal(pdx.to_array(x.shape), rdx)
+        np.testing.assert_array_equal(pdw.to_array(w.shape), rdw)
+        np.testing.assert_array_equal(pdb.to_array((F,)), dy.sum((0, 2, 3)))
 
 
 @pytest.mark.parametrize("case", [c for c in CASES if c[0] in ("px65", "c96", "s2_odd", "tiles_256", "one_pixel", "stem_odd", "stem_c4_k8")],
