@@ -366,21 +366,23 @@ inline bool pair_fits(const Plan& pl1, int M1, int N1, const Plan& pl2, int M2, 
            pl2.splits == 1 && tile_count(pl1.tile, M1, N1) + tile_count(pl2.tile, M2, N2) <= kNumCUs;
 }
 
-// Plans of two independent GEMMs (a backward's dA and dB). When their best
-// plans do not pair and one of them is a 32x32 plan, both retry on 64x64
-// tiles (one launch costs less than the smaller tile saves); returns whether
-// the plans pair, and leaves each GEMM's own best plan when they do not.
+// Plans of two independent GEMMs (a backward's dA and dB); returns whether they
+// pair, and leaves each GEMM's own best plan when they do not. Plans that pair
+// without a split over K stay together: their long chains run side by side, where
+// split 128x128 tiles would make three or four launches (backward of 3584 x 2752
+// x 128 27 against 41 us, 4288 x 4288 x 64 31 / 41). When the best plans do not pair
+// and one of them is a 32x32 plan, both retry on 64x64 tiles (one launch costs
+// less than the smaller tile saves).
 inline bool pair_plans(int M1, int N1, int K1, int M2, int N2, int K2, Plan& pl1, Plan& pl2) {
+    for (const bool t : {true, false}) {
+        pl1 = plan_tiles(M1, N1, K1, true, true, true, t, 0);
+        pl2 = plan_tiles(M2, N2, K2, true, true, true, t, 0);
+        if (pair_fits(pl1, M1, N1, pl2, M2, N2)) return true;
+        if (pl1.tile != Tile::T && pl2.tile != Tile::T) break;
+    }
     pl1 = plan_tiles(M1, N1, K1, true, true, true, true, kWidePartials);
     pl2 = plan_tiles(M2, N2, K2, true, true, true, true, kWidePartials);
-    if (pair_fits(pl1, M1, N1, pl2, M2, N2)) return true;
-    if (pl1.tile != Tile::T && pl2.tile != Tile::T) return false;
-    const Plan q1 = plan_tiles(M1, N1, K1, true, true, true, false);
-    const Plan q2 = plan_tiles(M2, N2, K2, true, true, true, false);
-    if (!pair_fits(q1, M1, N1, q2, M2, N2)) return false;
-    pl1 = q1;
-    pl2 = q2;
-    return true;
+    return pair_fits(pl1, M1, N1, pl2, M2, N2);
 }
 
 // Runs two independent problems: in one launch when pair_fits (the
