@@ -17,6 +17,7 @@
 #include "conv_band.h"
 #include "conv_packed.h"
 #include "conv_pointwise.h"
+#include "conv_routes.h"
 #include "gather.h"
 #include "kernels.h"
 #include "plan.h"
@@ -381,108 +382,11 @@ __global__ __launch_bounds__(256) void d2s_weights(const float* __restrict__ dW2
     dW[e] = dW2[((f * C2 + c2) * T2 + (r >> 1)) * U2 + (q >> 1)];
 }
 
-// Whether a stride-2 convolution takes the space-to-depth form: a kernel with
-// more taps than the direct band kernels hold (16) whose halves fit them.
-bool s2d_applies(int R, int S, int sh, int sw) {
-    return sh == 2 && sw == 2 && R * S > 16 && ((R + 1) / 2) * ((S + 1) / 2) <= 16;
-}
-
 unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 8192); }
 
 }  // namespace
 
 namespace {
-
-// Whether a pass runs on operands packed to fp16 (conv_packed.hip) or on the
-// kernels that read fp32 NCHW rows directly (conv_band.hip and the streaming
-// kernels). Packing costs one pass over the operands and pays where the direct
-// kernels read every value several times over (many filters), have few blocks
-// (many channels on small images), widen rows that are not float4s first, or
-// miss their fast shapes; it does not where a layer of few channels on large
-// aligned images is bound by reading its input once. Measured direct -> packed,
-// us, N x C x H x W -> F:
-//   3x3 s1  64x256x14x14 -> 256  fwd 68 -> 33, bwd 151 -> 66
-//           64x512x7x7 -> 512    fwd 67 -> 38, bwd 224 -> 76
-//           64x128x32x32 -> 128  fwd 68 -> 38, bwd 116 -> 98
-//           64x64x56x56 -> 128   fwd 51 -> 80, bwd 131 -> 175 (direct)
-//           64x128x32x32 -> 64   fwd 38 -> 29, bwd 62 -> 71 (bwd direct)
-//           64x32x8x8 -> 64      fwd 13 -> 13, bwd 36 -> 19
-//   3x3 s2  64x128x28x28 -> 256  fwd 43 -> 27, bwd 117 -> 61
-//   1x1     64x256x16x16 -> 256  fwd 37 -> 19, bwd 101 -> 36
-//           64x128x56x56 -> 64   fwd 56 -> 64, bwd 96 -> 104 (direct)
-//   5x5 s1  32x64x28x28 -> 64    fwd 164 -> 23, bwd 569 -> 54
-// The space-to-depth form of a first layer (few channels, large kernel, stride
-// 2) keeps its own path below.
-bool s2d_layer(int C, int R, int S, int sh, int sw) { return s2d_applies(R, S, sh, sw) && C <= 8; }
-
-bool packed_fwd_pays(int C, int W, int F, int R, int S, int sh, int sw, int ph, int pw) {
-    if (s2d_layer(C, R, S, sh, sw)) return false;
-    // 4 x 4 at stride 2 has a direct kernel (conv_stride2.hip): 32x64x16x16 ->
-    // 64 11 -> 16 us; other channel counts 16x128x64x64 -> 128 58 -> 32.
-    if (R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && (C == 32 || C == 64) && W % 4 == 0)
-        return false;
-    // Channels that are not a multiple of 8 (first layers): 39x3x28x28 -> 32
-    // 26 -> 13, 8x3x224x224 -> 64 71 -> 50.
-    if (W % 4 != 0 || C % 8 != 0 || R * S > 16 || sh > 1 || sw > 1) return true;
-    if (R * S == 1) return F >= 128 && (int64_t)C * F >= 128 * 128;
-    return C > 64;
-}
-
-bool packed_bwd_pays(int B, int C, int H, int W, int F, int R, int S, int sh, int sw, int ph, int pw) {
-    if (s2d_layer(C, R, S, sh, sw)) return false;
-    const int Wo = (W + 2 * pw - S) / sw + 1;
-    const int64_t pixels = (int64_t)B * H * W;
-    if (W % 4 != 0 || Wo % 4 != 0 || R * S > 16) return true;
-    // Few pixels: the direct kernels leave most CUs without a block, whatever
-    // the channels (16x32x32x32 -> 32 36 -> 24; at 64x64x28x28 -> 64, 50 k
-    // pixels, 41 -> 43). Channels not a multiple of 8: 111x3x28x28 -> 8 (87 k)
-    // 52 -> 44, 110x3x64x64 -> 8 80 -> 110.
-    if (pixels < 40000 || (C % 8 != 0 && pixels < 100000)) return true;
-    // (4 x 4 at stride 2, direct: conv_phase2.hip and conv_wgrad_s2.hip;
-    // 16x128x64x64 -> 128 50 -> 57)
-    if (R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && F % 32 == 0 && F <= 128 && W % 8 == 0)
-        return false;
-    if (sh > 1 || sw > 1) return true;
-    if (R * S == 1) return F >= 128;
-    return C >= 128 && F >= 128;
-}
-
-// 1x1 stride-1 layers in one pass over fp32 memory (conv_pointwise.hip), which
-// takes up to 128 filters (backward 64): the blocks stream tiles of 128 pixels,
-// and a long contraction on few tiles leaves CUs without one. Measured, us, with
-// the rules below -> in one pass:
-//   fwd  64x256x56x56 -> 64 (1600 tiles)  79 -> 62    64x128x56x56 -> 96  91 -> 54
-//        64x64x56x56 -> 64   34 -> 27     32x256x28x28 -> 64 (224)  28 -> 18
-//        32x128x28x28 -> 64 (224)  11.1 -> 11.7 (not)   32x256x14x14 -> 64 (64)  12 -> 16 (not)
-//        32x64x56x56 -> 96 (800)  25 -> 26 (not)        64x192x28x28 -> 80 (448)  30 -> 27
-//   bwd  64x256x56x56 -> 64  168 -> 126   64x64x28x28 -> 32 (448)  36 -> 20
-//        16x64x28x28 -> 64 (112)  18 -> 13              64x128x28x28 -> 64 (448)  39 -> 30
-//        32x256x28x28 -> 64 (224)  32 -> 39 (not)       256x256x14x14 -> 64 (512)  59 -> 64 (not)
-int64_t pixel_tiles(int B, int H, int W) { return (int64_t)B * (((int64_t)H * W + 127) / 128); }
-
-bool pointwise_fwd_pays(int B, int C, int H, int W, int F) {
-    if (F >= 128 && (int64_t)C * F >= 128 * 128) return false;  // packed
-    const int64_t tiles = pixel_tiles(B, H, W);
-    if (F > 64) return tiles >= 1200 || (C > 128 && tiles >= 400);
-    return C <= 64 || tiles >= 800 || (C > 128 && tiles >= 200);
-}
-
-bool pointwise_bwd_pays(int B, int C, int H, int W) { return C <= 128 || pixel_tiles(B, H, W) >= 800; }
-
-// ConvTranspose2D of 4 x 4 at stride 2 keeps its direct kernels
-// (conv_phase2.hip, conv_stride2.hip) on the channel counts they take:
-// 64x128x28x28 -> 64 fwd 33 -> 55, bwd 76 -> 79; others 64x256x14x14 -> 128
-// fwd 55 -> 40, bwd 161 -> 67; 2 x 2 16x128x16x16 -> 64 fwd 24 -> 12.
-bool packed_convT_fwd_pays(int F, int Wi, int W, int H, int R, int S, int sh, int sw) {
-    if (Wi % 4 != 0) return true;
-    if (sh == 1 && sw == 1) return F > 64;
-    return !(R == 4 && S == 4 && sh == 2 && sw == 2 && F % 32 == 0 && F <= 128 && H % 2 == 0 && W % 8 == 0);
-}
-
-bool packed_convT_bwd_pays(int F, int Wi, int C, int W, int R, int S, int sh, int sw, int ph, int pw) {
-    return Wi % 4 != 0 || W % 4 != 0 ||
-           !(R == 4 && S == 4 && sh == 2 && sw == 2 && ph == 1 && pw == 1 && (C == 32 || C == 64) && F <= 192);
-}
 
 int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H, int W, int F,
                  int R, int S, int sh, int sw, int ph, int pw, const ConvEpi& epi,
@@ -500,7 +404,7 @@ int conv_fwd_epi(const float* X, const float* Wt, float* Y, int B, int C, int H,
         SEERA_TRY(pointwise_conv_fwd(X, Wt, Y, B, C, (int64_t)H * W, F, epi, st, &used));
         if (used) return SEERA_OK;
     }
-    if (packed_fwd_pays(C, W, F, R, S, sh, sw, ph, pw)) {
+    if (packed_fwd_pays(B, C, H, W, F, R, S, sh, sw, ph, pw)) {
         SEERA_TRY(packed_conv_fwd(X, Wt, Y, B, C, H, W, F, R, S, sh, sw, ph, pw, epi, st, &used));
         if (used) return SEERA_OK;
     }
@@ -723,7 +627,7 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
     const int Ho = (H + 2 * ph - R) / sh + 1, Wo = (W + 2 * pw - S) / sw + 1;
     if ((int64_t)B * H * W <= 0x7fffffff && (int64_t)B * Ho * Wo <= 0x7fffffff) {
         bool packed = false, fused = false;
-        if (B > 0) {
+        if (B > 0 && packed_stem_bwd_pays(B, C, H, W, F, Wo)) {
             SEERA_TRY(packed_stem_bwd(dY, Wconv, X, dX, dW, db, B, C, H, W, F, R, S, sh, sw, ph, pw, st, &packed));
             if (packed) return SEERA_OK;
         }
@@ -747,7 +651,7 @@ int conv_bwd(const float* dY, const float* Wconv, const float* X, float* dX, flo
 int convT_fwd(const float* X, const float* Wt, float* out, int B, int F, int Hi, int Wi, int C, int H,
               int W, int R, int S, int sh, int sw, int ph, int pw, hipStream_t st) {
     bool used = false;
-    if (B > 0 && packed_convT_fwd_pays(F, Wi, W, H, R, S, sh, sw)) {
+    if (B > 0 && packed_convT_fwd_pays(B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw)) {
         SEERA_TRY(packed_convT_fwd(X, Wt, out, B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw, st, &used));
         if (used) return SEERA_OK;
     }
@@ -758,7 +662,7 @@ int convT_bwd(const float* dY, const float* Wt, const float* X, float* dX, float
               int Hi, int Wi, int C, int H, int W, int R, int S, int sh, int sw, int ph, int pw,
               hipStream_t st) {
     bool used = false;
-    if (B > 0 && packed_convT_bwd_pays(F, Wi, C, W, R, S, sh, sw, ph, pw)) {
+    if (B > 0 && packed_convT_bwd_pays(B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw)) {
         SEERA_TRY(packed_convT_bwd(dY, Wt, X, dX, dW, B, F, Hi, Wi, C, H, W, R, S, sh, sw, ph, pw, st, &used));
         if (used) return SEERA_OK;
     }

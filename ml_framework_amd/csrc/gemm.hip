@@ -10,8 +10,8 @@
 //                           from A; split-K with a deterministic reduce
 // No transposed copies and no host loop.
 #include <algorithm>
-#include <cmath>
 
+#include "gemm_routes.h"
 #include "kernels.h"
 #include "plan.h"
 
@@ -416,57 +416,6 @@ __global__ __launch_bounds__(256) void transpose_tiles4(const float* __restrict_
     }
 }
 
-// The share of the chip's 256 CUs that have work over the rounds of 256x256
-// tiles of an M x N result.
-double tile_fill(int M, int N) {
-    const double t = (double)((M + 255) / 256) * ((N + 255) / 256);
-    return t / (256.0 * std::ceil(t / 256.0));
-}
-
-// Whether an M x N product with float4-aligned rows that reads its operands
-// `reuse` times over is better off packed (below): the 256x256 tiles of the
-// streaming kernel leave CUs idle in their last round.
-bool tiles_leave_idle(int M, int N, double reuse) {
-    const double fill = tile_fill(M, N);
-    return (int64_t)((M + 255) / 256) * ((N + 255) / 256) > 256 ? fill < 0.8 && reuse >= 600
-                                                                : fill < 0.6 && reuse >= 1250;
-}
-
-// Whether a call runs on operands packed to fp16 (gemm_packed.hip). Reuse: the
-// multiply-adds per value packed. Measured without -> with (us, M x N x K; dA and dB in brackets):
-//  - rows that are not whole float4s, from kPackMin* multiply-adds on: below,
-//    the packing launch costs what it saves (332 x 539 x 103: 7.2 -> 8.8; 65 x
-//    4000 x 65 [15.4 -> 16.5]), and from a reuse of 12 [80] on (3 x 100001 x 101:
-//    18 -> 22; 16 x 4001 x 4001: 36 -> 29; 33 x 9001 x 2001: 54 -> 34 [reuse 65,
-//    76 -> 81]; 85 x 3687 x 2236 [reuse 160, 171 -> 34]); 511^3: 15.6 -> 9.7 [23.9 ->
-//    15.0], 3001 x 2047 x 1501: 60 -> 38 [141 -> 79], 4095^3: 190 -> 175 [378 -> 335].
-//  - a contraction that is not whole 32-deep slices, where the kernel cannot
-//    stream: with a reuse of 600 on (1000^3, reuse 500: 13.2 -> 14.8 [reuse 667,
-//    26.8 -> 25.1]; 1200^3: 22 -> 18 [46 -> 29]; 16384 x 512 x 500: 27 -> 32;
-//    100000 x 256 x 252: 63 -> 80 [reuse 253, 133 -> 191]).
-//  - tiles_leave_idle: 2560^3: 65 -> 54 [141 -> 105], 4608^3: 338 -> 240, 6144^3:
-//    759 -> 515 [1884 -> 995]; not 4096^3 (144 -> 167), 3584^3 (125 -> 131) or
-//    4096 x 11008 x 4096 (412 -> 438), whose tiles fill their rounds.
-constexpr double kPackMinFwd = 3e7, kPackMinBwd = 2e7;
-
-bool packed_fwd_pays(const void* A, const void* B, int M, int N, int K) {
-    const double macs = (double)M * N * K;
-    if (macs < kPackMinFwd) return false;
-    const double reuse = 1.0 / (1.0 / M + 1.0 / N);
-    if (K % 4 != 0 || N % 4 != 0 || !aligned16(A) || !aligned16(B)) return reuse >= 12;
-    if (K % 32 != 0) return reuse >= 600;
-    return tiles_leave_idle(M, N, reuse);
-}
-
-bool packed_bwd_pays(const void* A, const void* B, const void* dC, int M, int N, int K) {
-    const double macs = (double)M * N * K;
-    if (macs < kPackMinBwd) return false;
-    const double reuse = 2.0 / (1.0 / M + 1.0 / N + 1.0 / K);
-    if (K % 4 != 0 || N % 4 != 0 || !aligned16(A) || !aligned16(B) || !aligned16(dC)) return reuse >= 80;
-    if (M % 32 != 0 || N % 32 != 0) return reuse >= 600;
-    return tiles_leave_idle(M, K, reuse) || tiles_leave_idle(K, N, reuse);
-}
-
 }  // namespace
 
 int gemm_fwd(const float* A, const float* B, float* C, int M, int N, int K, int Nbatch,
@@ -474,7 +423,7 @@ int gemm_fwd(const float* A, const float* B, float* C, int M, int N, int K, int 
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
     bool used = false;
-    if (packed_fwd_pays(A, B, (int)Mb, N, K))
+    if (packed_gemm_fwd_pays(aligned16(A), aligned16(B), (int)Mb, N, K))
         SEERA_TRY(packed_gemm_fwd(A, B, nullptr, C, nullptr, (int)Mb, N, K, kActNone, false, st, &used));
     if (used) return SEERA_OK;
     // A [Mb, K] row-major (K-contiguous), B [K, N] row-major (N-contiguous).
@@ -486,7 +435,7 @@ int gemm_fwd_bias_act(const float* A, const float* B, const float* bias, float* 
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
     bool used = false;
-    if (packed_fwd_pays(A, B, (int)Mb, N, K))
+    if (packed_gemm_fwd_pays(aligned16(A), aligned16(B), (int)Mb, N, K))
         SEERA_TRY(packed_gemm_fwd(A, B, bias, C, mask, (int)Mb, N, K, act, true, st, &used));
     if (used) return SEERA_OK;
     Epi e;
@@ -501,7 +450,7 @@ int gemm_bwd_relu(const float* A, const float* B, const float* dC, const float* 
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
     bool used = false;
-    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+    if (packed_gemm_bwd_pays(aligned16(A), aligned16(B), aligned16(dC), (int)Mb, N, K))
         SEERA_TRY(packed_gemm_bwd(A, B, dC, mask, dA, dB, nullptr, (int)Mb, N, K, st, &used));
     if (used) return SEERA_OK;
     Epi e;
@@ -558,7 +507,7 @@ int gemm_bwd(const float* A, const float* B, const float* dC, float* dA, float* 
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
     bool used = false;
-    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+    if (packed_gemm_bwd_pays(aligned16(A), aligned16(B), aligned16(dC), (int)Mb, N, K))
         SEERA_TRY(packed_gemm_bwd(A, B, dC, nullptr, dA, dB, nullptr, (int)Mb, N, K, st, &used));
     if (used) return SEERA_OK;
     // dA [Mb, K] = dC [Mb, N] . B^T : B^T element (k, n) = B[k*N + n] is
@@ -575,7 +524,7 @@ int gemm_bwd_bias(const float* A, const float* B, const float* dC, const float* 
     const int64_t Mb = (int64_t)M * Nbatch;
     if (Mb > 0x7fffffff) return fail(SEERA_ERR_INVALID_ARGUMENT, "Nbatch*M exceeds int range");
     bool used = false;
-    if (packed_bwd_pays(A, B, dC, (int)Mb, N, K))
+    if (packed_gemm_bwd_pays(aligned16(A), aligned16(B), aligned16(dC), (int)Mb, N, K))
         SEERA_TRY(packed_gemm_bwd(A, B, dC, mask, dA, dB, db, (int)Mb, N, K, st, &used));
     if (used) return SEERA_OK;
     // dB [K, N] = A^T . dC with db[n] = sum_m dC[m, n] taken from the same
