@@ -304,7 +304,8 @@ enum PackedKind { kPlain, kS2dForward, kS2dInput };
 // One sum of a space-to-depth product over the kernel's own taps. The matrix
 // cores also multiply the added taps' zero weights, and 0 * inf is NaN where an
 // infinite operand is no term of the output: a lane that finds NaN takes the sum
-// from here. n: output channel; pi, pj: the output pixel in the phase's grid.
+// from here, as far as it stays a number (where all operands are NaN the first
+// eight settle it). n: output channel; pi, pj: the output pixel in the phase's grid.
 template <int BK, PackedKind KIND>
 __device__ __forceinline__ float own_taps_sum(const PackedConvArgs& a, int b, int pi, int pj, int n) {
     const PackedPhase& ph = a.ph[0];
@@ -313,14 +314,19 @@ __device__ __forceinline__ float own_taps_sum(const PackedConvArgs& a, int b, in
     for (int cb = 0; cb < a.ncb; ++cb)
         for (int tap = 0; tap < taps; ++tap) {
             const int t = tap / ph.U, u = tap - t * ph.U;
-            const half_t* x = a.x + cb * (int64_t)a.plane + ph.x0 +
-                              (int64_t)(b * a.HpWp + (pi * a.ish + t) * a.Wp + pj * a.isw + u) * a.pix;
-            const half_t* w = a.w + ph.woff + ((int64_t)(cb * taps + tap) * a.N + n) * BK;
-            for (int k = 0; k < BK; ++k) {
-                // (the forward's slice is a kernel row: 4 columns of 2 x 2 x 4 channels)
-                const int c2 = KIND == kS2dForward ? k & 15 : n, col = KIND == kS2dForward ? k >> 4 : 3 - u;
-                const int row = KIND == kS2dForward ? t : ph.T - 1 - t;
-                if (2 * row + ((c2 >> 1) & 1) < a.R && 2 * col + (c2 & 1) < a.S) s += (float)x[k] * (float)w[k];
+            const half8* x = reinterpret_cast<const half8*>(
+                a.x + cb * (int64_t)a.plane + ph.x0 +
+                (int64_t)(b * a.HpWp + (pi * a.ish + t) * a.Wp + pj * a.isw + u) * a.pix);
+            const half8* w = reinterpret_cast<const half8*>(a.w + ph.woff + ((int64_t)(cb * taps + tap) * a.N + n) * BK);
+            for (int k = 0; k < BK / 8 && s == s; ++k) {
+                const half8 xv = x[k], wv = w[k];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    // (the forward's slice is a kernel row: 4 columns of 2 x 2 x 4 channels)
+                    const int c2 = KIND == kS2dForward ? j : n, col = KIND == kS2dForward ? k >> 1 : 3 - u;
+                    const int row = KIND == kS2dForward ? t : ph.T - 1 - t;
+                    if (2 * row + ((c2 >> 1) & 1) < a.R && 2 * col + (c2 & 1) < a.S) s += (float)xv[j] * (float)wv[j];
+                }
             }
         }
     return s;
