@@ -14,6 +14,7 @@
 // A, B and dC once for both of its products (3001 x 2047 x 1501: 141 -> 79 us).
 // Reference: engine_cuda/src/GEMM.cu:13-103, 164-225.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "half_tile.h"
@@ -252,35 +253,40 @@ hipError_t launch_packed_gemm(PackedGemmArgs g, int splits, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Tile and splits of an M x N product of `slices` 64-deep slices. Time per slice
-// (measured with the operands in L2): 256x128 0.64 us with one block per CU,
-// which the matrix cores bound; 128x128 0.40 us with one block per CU, bound by LDS
-// (1.5 cycles of LDS per matrix-core cycle, against 1.1); 64x64 0.32 us with
-// three blocks per CU. 4097^3: 128x128 257 us, 256x128 214 us; 2000^3: 35 us and
-// 40 us; 511^3: 64x64.
+// Tile and splits of an M x N product of `slices` 64-deep slices, from times over
+// 73 shapes of 64 to 16385 rows with every tile and 1 to 16 splits (us, a fit within
+// 10 % on average). A block takes a start-up (first loads, stores) and its slices:
+//   256x128  8.7 + 0.71 a slice, one per CU, bound by the matrix cores
+//   128x128  4.9 + 0.47 a slice, one per CU, bound by LDS (1.5 cycles of it per
+//            matrix-core cycle, against 1.1)
+//   64x64    2.1 + 0.35, 0.44 or 0.54 a slice with one, two or three on a CU
+// and a split adds 2.8 (a launch) and a pass over the partials at 3.1 TB/s. The chosen tile,
+// us with the packing: 4097^3 256x128 214 (128x128 223, 64x64 266), 3001x2047x1501 256x128
+// 39 (64x64 43), 2047^3 128x128 35 (256x128 41), 1301^3 64x64 20 (128x128 24); of 73 shapes
+// two lose more than 8 %: 795x1046x4432 35 (31), 1597x4059x379 25 (23).
 enum { kTile64, kTile128, kTile256 };
 struct PackedPlan {
     int tile, splits, sps;
     PackedPlan(int M, int N, int slices) : tile(kTile128), splits(1) {
         auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+        auto per_cu = [](int64_t blocks) { return (double)((blocks + 255) / 256); };
         double best = 1e30;
         for (int s = 1; s <= 32; s *= 2) {
             if (s > 1 && slices / s < 4) break;
-            // us: rounds of blocks, each a start-up and its slices; a split adds
-            // the reduce (a launch and a pass over the partials)
-            auto consider = [&](int t, int64_t n, double slice, int per_cu) {
-                const int64_t rounds = (n * s + 256 * per_cu - 1) / (256 * per_cu);
-                const double us = (double)rounds * (3.0 + slice * ((slices + s - 1) / s)) +
-                                  (s > 1 ? 5.0 + (double)s * M * N * 4 / 2.0e6 : 0.0);
+            const double n = (slices + s - 1) / s;
+            auto consider = [&](int t, double us) {
+                if (s > 1) us += 2.8 + (double)s * M * N * 4 / 3.1e6;
                 if (us < best) {
                     best = us;
                     tile = t;
                     splits = s;
                 }
             };
-            consider(kTile256, tiles(256, 128), 0.64, 1);
-            consider(kTile128, tiles(128, 128), 0.40, 1);
-            consider(kTile64, tiles(64, 64), 0.32, 3);
+            consider(kTile256, per_cu(tiles(256, 128) * s) * (8.7 + 0.71 * n));
+            consider(kTile128, per_cu(tiles(128, 128) * s) * (4.9 + 0.47 * n));
+            const double b = per_cu(tiles(64, 64) * s), full = std::floor(b / 3), rest = b - 3 * full;
+            consider(kTile64, (full + (rest > 0 ? 1 : 0)) * 2.1 +
+                                  n * (full * 0.54 + (rest == 1 ? 0.35 : rest == 2 ? 0.44 : 0.0)));
         }
         sps = (slices + splits - 1) / splits;
         splits = (slices + sps - 1) / sps;

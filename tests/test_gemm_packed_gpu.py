@@ -32,12 +32,13 @@ SHAPES = [
     (85, 511, 513, 3),     # 64, 64, 64 over a batch
     (1030, 66, 515, 1),    # 64 with one slice and two columns more
     (70, 4099, 130, 1),    # 64 in 16 parts, 64, 64
-    (1025, 8191, 333, 1),  # 128 in 8 parts, 256, 64
-    (2305, 1001, 3333, 1), # 64, 64, 128
-    (3329, 129, 2817, 1),  # 256, 64 in 4, 64 in 4
-    (300, 2561, 2561, 1),  # 64, 64, 256
+    (1025, 8191, 333, 1),  # 128 in 8 parts, 64, 64
+    (2305, 1001, 3333, 1), # 64, 128, 128
+    (3329, 129, 2817, 1),  # 64, 64 in 4, 64 in 4
+    (300, 2561, 2561, 1),  # 64 in 2, 64 in 2, 256
     (1500, 1500, 1500, 1), # whole float4s, ragged slices
     (2304, 2560, 2560, 1), # whole slices: tiles that leave compute units idle
+    (3001, 1501, 2047, 1), # 256, 256, 128
 ]
 
 
@@ -51,7 +52,7 @@ def test_exact(M, K, N, nb):
     np.testing.assert_array_equal(db, _mm(a.reshape(-1, K).T, dc.reshape(-1, N)))
 
 
-@pytest.mark.parametrize("M,K,N,nb", SHAPES[:8])
+@pytest.mark.parametrize("M,K,N,nb", SHAPES[:8] + SHAPES[-1:])
 def test_epilogues(M, K, N, nb):
     r = np.random.default_rng(N)
     a, b, dc = _ints(r, (nb, M, K)), _ints(r, (K, N)), _ints(r, (nb, M, N))
