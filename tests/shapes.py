@@ -70,9 +70,11 @@ CONV2D_STREAM = [
     # 64 channels on rows wider than 56: the three-role forward in column tiles
     ("s18", 1, 64, 6, 60, 64, 3, 3, 1, 1),     # 2 tiles of 32 (the second 28 wide)
     ("s19", 2, 64, 5, 200, 40, 3, 3, 1, 1),    # 4 tiles of 52 (the last 44), partial filter tile
-    # more than 64 channels on the three-role kernel: one launch per
-    # 64-channel slice, each after the first adding to the output (up to 4
-    # slice x filter-tile launches, two filter tiles on rows of 56 or more)
+    # more than 64 channels on aligned rows: operands packed to fp16 at these
+    # sizes; without staging memory (test_unstaged_gpu.py), and on far larger
+    # images, the three-role kernel, one launch per 64-channel slice, each after
+    # the first adding to the output (up to 4 slice x filter-tile launches, two
+    # filter tiles on rows of 56 or more)
     ("m01", 2, 128, 12, 16, 64, 3, 3, 1, 1),   # forward in 2 slices
     ("m02", 1, 192, 6, 60, 64, 3, 3, 1, 1),    # 3 slices, column tiles
     ("m03", 2, 64, 8, 8, 128, 3, 3, 1, 1),     # dX over 128 dY channels: 2 slices
@@ -94,9 +96,8 @@ CONV2D_EDGE = [
     ("e06", 2, 24, 12, 16, 40, 1, 7, 1, 0),
     ("e07", 2, 8, 6, 6, 8, 3, 3, 1, 2),
     ("e08", 1, 65, 9, 9, 129, 3, 3, 2, 1),
-    # rows that are not a multiple of 4 floats: the band and row-streaming
-    # kernels on copies widened with zero columns (X for the forward, dY for
-    # dX, both for dW)
+    # rows that are not a multiple of 4 floats: operands packed to fp16 (on a
+    # stream without staging memory the gather GEMMs: test_unstaged_gpu.py)
     ("e09", 2, 64, 14, 14, 64, 3, 3, 1, 1),    # 14x14 (a ResNet stage)
     ("e10", 2, 256, 7, 7, 48, 3, 3, 1, 1),     # 7x7, 8 channel chunks, partial filter tile
     ("e11", 2, 128, 28, 28, 64, 3, 3, 2, 1),   # stride 2: dY rows of 14
@@ -108,10 +109,11 @@ CONV2D_EDGE = [
     ("k02", 2, 64, 7, 8, 256, 1, 1, 1, 0),     # 256 filters
     ("k03", 2, 30, 6, 10, 18, 1, 1, 1, 0),     # channels not a multiple of 8
     # stride 2 with more than 16 taps: the space-to-depth form (4C channels,
-    # ceil(R/2) x ceil(S/2) taps, stride 1)
-    ("d01", 2, 3, 20, 24, 8, 7, 7, 2, 3),      # a 7x7 stem: all three passes in that form
-    ("d02", 2, 5, 17, 21, 16, 5, 5, 2, 2),     # 5x5, 11-column output: forward only
-    ("d03", 1, 20, 12, 16, 70, 7, 7, 2, 3),    # 80 channels in that form (3 chunks), 2 filter tiles
+    # ceil(R/2) x ceil(S/2) taps, stride 1) up to 8 channels, packed up to 4
+    ("d01", 2, 3, 20, 24, 8, 7, 7, 2, 3),      # a 7x7 stem, packed
+    ("d02", 2, 5, 17, 21, 16, 5, 5, 2, 2),     # 5x5, 11-column output: the forward on fp32 copies
+    ("d03", 1, 20, 12, 16, 70, 7, 7, 2, 3),    # 20 channels: an ordinary packed layer of 49 taps
+    ("d04", 2, 6, 20, 24, 40, 7, 7, 2, 3),     # 6 channels: all three passes on fp32 copies
 ]
 
 # Stride-2 shapes for the four-phase and column-parity kernels (not from the
@@ -173,14 +175,14 @@ CONVT = [
 # Transposed shapes for the four-phase kernel (not from the reference's
 # tests): one and three input-channel chunks, 36 phase columns (two column
 # tiles), 40 output channels (a partial 32-filter tile), a 2x2 kernel; and
-# input rows of 7 and 9 columns (the widened-copy path).
+# input rows of 7 and 9 columns (packed operands).
 CONVT_PHASE2 = [
     ("u01", 2, 32, 6, 20, 40, 4, 4, 2, 1),
     ("u02", 2, 96, 10, 36, 24, 4, 4, 2, 1),
     ("u03", 3, 64, 8, 8, 16, 2, 2, 2, 0),
     ("u04", 1, 128, 28, 28, 64, 4, 4, 2, 1),   # one image of config 5
     ("u05", 2, 96, 14, 20, 32, 4, 4, 2, 1),    # dX by column-parity streaming, one chunk
-    ("u06", 2, 64, 7, 7, 32, 4, 4, 2, 1),      # 7-column input rows (widened copy)
+    ("u06", 2, 64, 7, 7, 32, 4, 4, 2, 1),      # 7-column input rows
     ("u07", 2, 32, 5, 9, 16, 3, 3, 2, 1),      # 3x3 s2, odd widths both ways
 ]
 

@@ -27,13 +27,13 @@ SHAPES = [
     ("stream3x3", 4, 64, 56, 56, 64, 3, 1, 1),    # config 4's kernel at batch 4
     ("stream_2ft", 2, 96, 20, 20, 80, 3, 1, 1),     # 2 filter tiles, 80 filters
     ("stream5x5", 3, 16, 24, 24, 24, 5, 1, 2),
-    ("band_s2", 8, 32, 64, 64, 64, 3, 2, 1),       # strided: band kernel
-    ("band_2x2s2", 4, 32, 32, 32, 64, 2, 2, 0),    # 4 taps, small band
-    ("gather_w10", 2, 3, 10, 10, 4, 5, 2, 2),      # width % 4 != 0: gather GEMM
+    ("band_s2", 8, 32, 64, 64, 64, 3, 2, 1),       # strided: packed operands
+    ("band_2x2s2", 4, 32, 32, 32, 64, 2, 2, 0),    # 4 taps, packed operands
+    ("gather_w10", 2, 3, 10, 10, 4, 5, 2, 2),      # 5x5 stride 2 on 3 channels: fp32 space-to-depth copies
     ("gather_1f", 4, 8, 9, 9, 1, 3, 1, 1),         # one filter
     ("conv1x1", 3, 32, 10, 12, 24, 1, 1, 0),       # 1x1 projection
-    ("s2d_7x7", 2, 3, 16, 16, 8, 7, 2, 3),         # 7x7 s2: space-to-depth form
-    ("slices_128", 2, 128, 10, 12, 70, 3, 1, 1),   # 2 channel slices: epilogue on the total
+    ("s2d_7x7", 2, 3, 16, 16, 8, 7, 2, 3),         # 7x7 s2: space-to-depth form, packed
+    ("slices_128", 2, 128, 10, 12, 70, 3, 1, 1),   # 2 channel blocks: epilogue on the total
 ]
 
 
@@ -138,8 +138,9 @@ def test_fused_conv_against_oracle(case, act):
         assert np.array_equal(mask[clear], (pre[clear] > 0).astype(np.float32))
 
 
-# (name, N, C, H, W, F, K, stride, pad): band_s2 and gather_w10 fall back to
-# a separate db pass; the others take db from the dW pass's loads of dY.
+# (name, N, C, H, W, F, K, stride, pad): gather_w10 falls back to a separate db
+# pass; packed layers take db from the packing pass's loads of dY, the others
+# from the dW pass's.
 BWD_BIAS = [
     ("stream3x3_cfg4_b4", 4, 64, 56, 56, 64, 3, 1, 1),
     ("stream3x3_2tiles", 3, 128, 20, 20, 96, 3, 1, 1),    # two filter and channel tiles

@@ -151,8 +151,8 @@ def test_matmul_bwd_parity(M, K, N, nb):
 
 
 # Large GEMMs whose operands are not vector-aligned, or whose K is not a
-# whole number of 32-deep slices, run on zero-padded staging copies of both
-# operands (odd everything; aligned with K % 32 != 0; a folded batch).
+# whole number of 32-deep slices, run on operands packed to fp16 (odd
+# everything; aligned with K % 32 != 0; a folded batch).
 PADDED = [(2049, 2047, 1025, 1), (1024, 4100, 1024, 1), (700, 2051, 1001, 3)]
 
 

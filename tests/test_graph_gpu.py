@@ -336,9 +336,9 @@ def test_convT_backward_graph(lib, stream):
 
 def test_staged_layouts_graph(lib, stream):
     """Convolutions that stage a re-laid-out operand in the second per-stream
-    buffer: a 14x14 layer (rows widened to 16 floats for the forward, dX and
-    dW) and a 7x7 stride-2 stem (space-to-depth) forward and backward, with
-    bias and ReLU on the stem, captured and replayed."""
+    buffer: a 14x14 layer and a 7x7 stride-2 stem (space-to-depth), both on
+    operands packed to fp16, forward and backward, with bias and ReLU on the
+    stem, captured and replayed."""
     r = np.random.default_rng(5)
     N, C, H, W, F = 4, 64, 14, 14, 64
     x = DeviceBuffer(N * C * H * W * 4)

@@ -1,8 +1,8 @@
 """Conv2D, ConvTranspose2D and GEMM forward/backward on seeded random shapes (not
 from the reference's tests): channel counts, sizes, kernels, strides and
 paddings drawn over ranges that reach every dispatch path (three-role and
-row-streaming kernels, channel slices, column tiles, widened rows, stride
-phases, space-to-depth, the band and gather kernels), each against the oracle
+row-streaming kernels, column tiles, packed operands, stride phases,
+space-to-depth, the band kernels), each against the oracle
 at the tolerance of test_conv_gpu.py. The draws are fixed by the seed."""
 import zlib
 
@@ -121,7 +121,7 @@ GEMM_CASES = _gemm_cases(20, 20261204)
 @pytest.mark.parametrize("case", GEMM_CASES, ids=[c[0] for c in GEMM_CASES])
 def test_matmul_random_shape(case):
     """Seeded random GEMM shapes (every tile kernel, split-K, wave groups,
-    pairs, scalar loads and the padded staging copies), forward and backward."""
+    pairs, scalar loads and operands packed to fp16), forward and backward."""
     from tests.helpers import hip_matmul, hip_matmul_bwd
     name, M, K, N, nb = case
     r = np.random.default_rng(zlib.crc32(repr(case).encode()))
@@ -231,7 +231,7 @@ def test_conv2d_epilogues_random_shape(case):
 
 # The specialised kernels of the configs' layer types on random geometry:
 # 3x3 stride-1 pad-1 convolutions of multiples of 64 channels (three-role
-# forward, one-pass backward, channel slices, column tiles, widened rows) and
+# forward, one-pass backward, column tiles, packed operands) and
 # 4x4 stride-2 pad-1 transposed convolutions (phase and stride-2 streaming
 # kernels), with random batch, height and width.
 def _hot_conv_cases(n, seed):

@@ -1,7 +1,8 @@
 """Calls whose operands would be packed to fp16 or widened, on a stream that has
 no memory for the copies: captured before any call of their size, so the staging
 buffer cannot grow, they run on the kernels that read the caller's tensors
-(gather GEMMs for convolutions, scalar-load tiles for products). Each graph is
+(gather GEMMs and, on aligned rows, the band and channel-slice kernels for
+convolutions; scalar-load tiles for products). Each graph is
 replayed with other work between the replays, and every replay is compared with
 the oracle; a call made outside capture afterwards takes the copies and must
 agree within the order of its sums."""
@@ -14,12 +15,12 @@ import oracle
 from ml_framework_amd import capi
 from ml_framework_amd.capi import DeviceBuffer
 from oracle import fp16r
-from tests.helpers import assert_parity, convT_hw, out_hw
+from tests.helpers import assert_parity, convT_hw, hip_conv_bwd, hip_conv_fwd, out_hw
 
 pytestmark = pytest.mark.gpu
 S = oracle.seera_cpp
-# fp32 sums of at most 2 thousand of the same fp16 products in two orders:
-# 2 * 0.41 * 2^-24 * sqrt(1000) = 1.5e-6 of the result (see test_conv_packed_gpu.py)
+# fp32 sums of at most 2304 of the same fp16 products in two orders:
+# 2 * 0.41 * 2^-24 * sqrt(2304 / 2) = 1.7e-6 of the result (see test_conv_packed_gpu.py)
 STRICT = 5e-6
 
 
@@ -90,6 +91,12 @@ def _dev(a):
     (2, 16, 13, 15, 70, 3, 2, 1),    # stride 2
     (2, 20, 9, 10, 24, 5, 1, 2),     # 25 taps
     (2, 3, 30, 26, 33, 7, 2, 3),     # a first layer
+    (2, 128, 12, 16, 64, 3, 1, 1),   # two 64-channel slices, the epilogue on their total
+    (1, 192, 6, 60, 64, 3, 1, 1),    # three, column tiles
+    (1, 256, 5, 20, 64, 3, 1, 1),    # four
+    (1, 128, 6, 60, 96, 3, 1, 1),    # two slices x two filter tiles (the second partial)
+    (1, 128, 4, 64, 128, 3, 1, 1),
+    (2, 96, 10, 12, 40, 3, 2, 1),    # band kernels, aligned: stride 2
 ], ids=str)
 def test_conv2d(lib, N, C, H, W, F, K, s, p):
     r = np.random.default_rng(N + C + H)
@@ -135,3 +142,24 @@ def test_matmul(lib, M, K, N):
     _unstaged(lib, [("seera_hip_matmul_async", (pa.ptr, pb.ptr, pc.ptr, M, N, K, 1)),
                     ("seera_hip_matmul_bwd_async", (pa.ptr, pb.ptr, pdc.ptr, pda.ptr, pdb.ptr, M, N, K, 1))],
               [(pc, (M, N), c), (pda, (M, K), da[0]), (pdb, (K, N), db)])
+
+
+@pytest.mark.parametrize("N,C,H,W,F,K,s,p", [
+    (2, 24, 22, 30, 40, 3, 4, 1),    # 16 stride residues, rows widened to float4s for the forward and dW
+    (1, 16, 33, 41, 24, 5, 5, 2),    # 25 of them
+    (2, 6, 14, 15, 10, 9, 1, 4),     # 81 taps
+    (1, 12, 15, 20, 18, 9, 2, 4),
+], ids=str)
+def test_beyond_packed_sizes(lib, N, C, H, W, F, K, s, p):
+    """Strides and kernels that the packed convolutions do not hold (more than 9
+    residues, more than 64 taps)."""
+    r = np.random.default_rng(N + C + H)
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    w = (r.standard_normal((F, C, K, K)) / np.sqrt(C * K * K)).astype(np.float32)
+    y = S.conv2d_forward(fp16r(x), fp16r(w), s, s, p, p)
+    assert_parity(hip_conv_fwd(x, w, s, p), y, "fwd", STRICT)
+    dy = r.standard_normal(y.shape).astype(np.float32)
+    dx, dw = hip_conv_bwd(dy, x, w, s, p)
+    rdx, rdw = S.conv2d_backward(fp16r(dy), fp16r(x), fp16r(w), s, s, p, p)
+    assert_parity(dx, rdx, "dX", STRICT)
+    assert_parity(dw, rdw, "dW", STRICT)
