@@ -223,7 +223,11 @@ int seera_hip_transpose_3d(const float *in, float *out, int Nbatch, int M,
  * conv[b,n,ho,wo] = sum_{c,r,s} kernel[n,c,r,s] *
  *                   image[b,c,ho*stride_h-pad_h+r, wo*stride_w-pad_w+s]
  * image [batchN,C,H,W], kernel [N,C,R,S], conv [batchN,N,Hout,Wout],
- * Hout = (H + 2 pad_h - R)/stride_h + 1. */
+ * Hout = (H + 2 pad_h - R)/stride_h + 1.
+ * Infinite and NaN values reach the outputs they are terms of, in the forward
+ * and both gradients; at stride 2 with more than 16 taps on at most 8 channels
+ * (7 and 8 wide kernels: on 5 to 8) they may also make NaN of outputs beside
+ * those, since the kernel is rounded up to even extents with zeros there. */
 int seera_hip_conv2d_fwd(const float *image, const float *kernel, float *conv,
                          int batchN, int C, int H, int W, int N, int R, int S,
                          int pad_h, int pad_w, int stride_h, int stride_w);
